@@ -82,7 +82,8 @@ def kernel_work(rs, kernel, el, prec):
     '''Algorithmic bytes and MFMA flops (as issued) of one launch of a radial step kernel. Per grid point in FP32:
     k->r 28 B (the stage input in, E_r out: 16 B, plus 12 B of kz tables), source 16 B (E_r in, J_r out), r->k 52 B
     (J_r in and the RK stage: 40 B, plus the tables) over the columns of the nonlinear band only; 96 B per RHS in
-    all. FP64 doubles them. The contractions issue 4 N_cols Nk Nr flops, three times that in BF16x3.'''
+    all. An exchange does both contractions with one read of the state and tables: the r->k bytes and E_r out. FP64
+    doubles them. The contractions issue 4 N_cols Nk Nr flops, three times that in BF16x3.'''
     T = rs.field_tool.GetTransverseTool()
     nw, nr, nk = rs.N[0], rs.N[1], getattr(T, 'Nk', rs.N[1])
     scale = el / 4.0
@@ -92,6 +93,9 @@ def kernel_work(rs, kernel, el, prec):
     if kernel == 'hankel_r2k':
         f1 = nl_columns(rs)
         return 52.0 * scale * f1 * nk, 4.0 * f1 * nk * nr * issued
+    if kernel == 'exchange':
+        f1 = nl_columns(rs)
+        return scale * (52.0 * f1 * nk + 8.0 * nw * nr), 4.0 * (f1 + nw) * nk * nr * issued
     if kernel == 'source':
         return 16.0 * scale * nw * nr, 0.0
     return None, None
@@ -99,6 +103,7 @@ def kernel_work(rs, kernel, el, prec):
 
 KERNEL_NAMES = {'hankel': 'f_hankel k->r (MFMA contraction with the fused RK stage prologue)',
                 'hankel_r2k': 'f_hankel r->k (MFMA contraction with the fused RK stage epilogue)',
+                'exchange': 'f_exchange (r->k contraction of a stage with its RK epilogue, k->r of the next)',
                 'source': 'f_source (strip transforms, rate, density scan, Kerr and plasma current)'}
 
 
@@ -172,7 +177,7 @@ def pcie_inclusive(rs, prec, K):
     return rs.N[0] * rs.N[1] * n / (t1 - t0)
 
 
-CLASSES = ('hankel', 'hankel_r2k', 'source', 'point', 'reduce', 'transverse_fft')
+CLASSES = ('hankel', 'hankel_r2k', 'exchange', 'source', 'point', 'reduce', 'transverse_fft')
 
 
 def radial_measure(vol, prec, K, W, plain_steps, compare=True, counters=None, error_steps=None, module=uppe_kernel):

@@ -213,9 +213,10 @@ int uppe_get_info(uppe_handle* h, uppe_info* info);
  * enable != 0 starts recording and clears totals; uppe_profile_read returns total milliseconds and launch
  * count of a class. The radial transforms are two classes: UPPE_KC_HANKEL for the k->r direction (and the
  * one-off transforms of set_field and finish), UPPE_KC_HANKEL_R2K for the r->k direction with the RK stage
- * epilogue. */
+ * epilogue; UPPE_KC_EXCHANGE is both in one launch, the r->k direction of a stage and the k->r direction of the
+ * next. */
 enum { UPPE_KC_HANKEL = 0, UPPE_KC_SOURCE = 1, UPPE_KC_POINT = 2, UPPE_KC_REDUCE = 3, UPPE_KC_TRANSVERSE_FFT = 4,
-       UPPE_KC_HANKEL_R2K = 5, UPPE_KC_COUNT = 6 };
+       UPPE_KC_HANKEL_R2K = 5, UPPE_KC_EXCHANGE = 6, UPPE_KC_COUNT = 7 };
 int uppe_profile_enable(uppe_handle* h, int enable);
 int uppe_profile_read(uppe_handle* h, int kernel_class, double* total_ms, long long* launches);
 

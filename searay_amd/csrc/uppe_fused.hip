@@ -21,6 +21,7 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 
 namespace uppe {
 
@@ -144,6 +145,12 @@ struct FusedState {
   struct HkPlan {
     int tiles = 1, split = 1, nwv = 1, rt = 1, wide = 0;
   } plan[2];
+  // launch plan of the exchange (r2k of one stage and k2r of the next): complex columns of an nl tile and of a
+  // linear tile (wn = 0: no exchange for this grid), waves, 16-row tiles per wave
+  struct XPlan {
+    int wn = 0, wl = 0, nwv = 1, rt = 1;
+  } xplan;
+  bool cond_one = true;  // the conditioner is one in every column at and above f1
   int n_cu = 256;
   int spt = 0;          // source samples per thread of the step (0: the default shape)
   int tuned_f1 = -1;    // nonlinear band the contraction plans were timed for (-1: not yet)
@@ -160,6 +167,7 @@ struct FusedState {
   int ckq_cap = 0, ckst_cap = 0, ckqm_cap = 0;  // segments
   int zrec_cap = 0;                             // doubles (3 per step)
   bool recorded = false, er_last_valid = false;
+  bool rec_known = false;  // the recorded run's step sizes were known before its stages (fixed or replayed)
   void* ck_q = nullptr;
   StepState* ck_st = nullptr;
   unsigned long long* ck_qmax = nullptr;
@@ -1182,6 +1190,552 @@ __global__ __launch_bounds__(BN > 16 ? 512 : 1024) void f_hankel(
                                            blockIdx.z);
 }
 
+// DPP lane move (gfx9 control codes: quad_perm 1,0,3,2 = 0xB1, row_shr:n = 0x110 + n,
+// row_ror:n = 0x120 + n, wave_shr:1 = 0x138, row_bcast:15 = 0x142, row_bcast:31 = 0x143); lanes without a source, or in rows outside RM, read 0
+template <int CTRL, int RM, typename T>
+__device__ inline T dpp_move(T v) {
+  if constexpr (sizeof(T) == 4) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, RM, 0xf, false));
+  } else {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, RM, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, RM, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------
+// Exchange: the r2k contraction of one RK stage and the k2r contraction of the next in one launch
+//
+// The r2k epilogue of a column tile leaves the slope of exactly the columns whose next stage input that tile's k2r
+// contraction reads, so a workgroup that holds all rows of its columns goes from J_r to the next stage's E_r
+// without another launch and without reading q, kz and the phase table a second time. Phases of a tile:
+//   J_r slab -> LDS;  Hf . J;  per point: slope, RK bookkeeping, next stage input, linear propagation, E = i kz A;
+//   E slab -> LDS;  Hb . E;  store E_r.
+// Columns f >= f1 carry no current: their tiles ("linear" tiles, after the nl tiles) only form E_r from q. That E_r
+// depends on the phase coordinate alone, so a linear tile whose coordinate has not moved since the last stage (from
+// stage 2 to 3, and from stage 4 to the next step's stage 1 inside a subcycle) leaves it in place (keep).
+// Stages 1-4 are exchanges. The step size of an adaptive run is known only when every tile of stage 1 has left its
+// estimate, so such runs take stage 1 -> 2 as two launches: stage 1 with `est` ends after the points, and stage
+// X_OPEN2 starts with them. Stage X_OPEN opens a run: every tile only forms the first E_r, with the arithmetic and
+// the tiles of stage 4, so that a run resumed from a stored state repeats the run it resumes bit for bit.
+//
+// At the sizes of one radial grid a launch is a chain of latencies. The points are therefore worked on where the
+// matrix instruction leaves them (the lanes of a pair hold the real and imaginary part of the same points and share
+// them out), without a pass through LDS, and the step state, J, the points' operands and the operator's first
+// fragments are all requested before any of them is waited for.
+// ---------------------------------------------------------------------------------------------------
+enum { X_OPEN = 0, X_OPEN2 = 5 };
+
+// waves per workgroup: 16, and 8 in FP64, whose points (double sines and exponentials) need more than the 128
+// registers that 16 waves leave each
+constexpr int x_max_waves(int cm) { return cm == CM_F64 ? 8 : 16; }
+
+template <int CM>
+struct XArgs {
+  using T = typename MfmaTraits<CM>::T;
+  using C = cplx<T>;
+  using F = typename MfmaTraits<CM>::frag_t;
+  const F *fhi, *flo;  // Hf (r2k), nk x nr
+  const F *bhi, *blo;  // Hb (k2r), nr x nk
+  const C* jr;
+  C* er;
+  const double* phs;
+  const C* kzc;
+  const T* cond;
+  C *q, *k1, *k2, *k3;
+  StepState* st;
+  unsigned long long *qmax, *qmax_next;
+  long zs;            // elements between the instances of a batched launch (or azimuthal modes), 0 for one grid
+  int nr, nk, kpf, kpb, row;  // kpf, kpb: padded contraction lengths over r and over k; row: elements per array row
+  int f1, nw, nlt;    // nonlinear band, columns, nl tiles (the first of the grid)
+  int wn, wl;         // complex columns of an nl and of a linear tile (powers of two)
+  int stage, est, env, zst, share;
+  int keep;           // bit 0: E_r is where the last stage left it, bit 1: the conditioner is one from f1 up
+};
+
+// How a tile's complex columns lie in the 16 real columns of a matrix product. X_WIDE: 8 complex columns, re and im
+// side by side. X_HALF: up to 4 in the lower 8 columns, the upper ones unused. X_PACK (BF16x3): up to 4, their hi
+// halves in the lower 8 columns and lo halves in the upper 8, so that two products (A_hi and A_lo with the packed
+// tile) give all four partial products.
+enum { X_WIDE = 0, X_HALF = 1, X_PACK = 2 };
+
+// LDS slab of a contraction's B operand, kp rows (k) of 16 real columns. BF16x3: columns of k-contiguous halves
+// (hi columns then lo columns, or both in one packed tile); others: [k][16].
+template <int CM>
+constexpr size_t x_slab_bytes(int kp) {
+  return CM == CM_BF16X3 ? (size_t)2 * 16 * (kp + 8) * 2 : (size_t)16 * kp * sizeof(typename MfmaTraits<CM>::T);
+}
+
+constexpr int x_lo_columns(int lay) { return lay == X_PACK ? 8 : 16; }  // from a hi column to its lo column
+
+// rows k and k + 1 (k even) of complex column cf of a slab
+template <int CM, int LAY>
+__device__ __forceinline__ void x_put2(char* slab, int kp, int k, int cf, cplx<typename MfmaTraits<CM>::T> v0,
+                                       cplx<typename MfmaTraits<CM>::T> v1) {
+  if constexpr (CM == CM_BF16X3) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const int ldb = kp + 8;
+    __bf16* hi = reinterpret_cast<__bf16*>(slab) + (2 * cf) * ldb + k;
+    __bf16* lo = hi + x_lo_columns(LAY) * ldb;
+    const bf16x2 hr = {(__bf16)v0.re, (__bf16)v1.re}, hm = {(__bf16)v0.im, (__bf16)v1.im};
+    *reinterpret_cast<bf16x2*>(hi) = hr;
+    *reinterpret_cast<bf16x2*>(hi + ldb) = hm;
+    *reinterpret_cast<bf16x2*>(lo) = bf16x2{(__bf16)(v0.re - (float)hr[0]), (__bf16)(v1.re - (float)hr[1])};
+    *reinterpret_cast<bf16x2*>(lo + ldb) = bf16x2{(__bf16)(v0.im - (float)hm[0]), (__bf16)(v1.im - (float)hm[1])};
+  } else {
+    using C = cplx<typename MfmaTraits<CM>::T>;
+    C* p = reinterpret_cast<C*>(slab) + k * 8 + cf;
+    p[0] = v0;
+    p[8] = v1;
+  }
+}
+
+// row k of complex column cf
+template <int CM, int LAY>
+__device__ __forceinline__ void x_put1(char* slab, int kp, int k, int cf, cplx<typename MfmaTraits<CM>::T> v) {
+  if constexpr (CM == CM_BF16X3) {
+    const int ldb = kp + 8;
+    __bf16* hi = reinterpret_cast<__bf16*>(slab) + (2 * cf) * ldb + k;
+    __bf16* lo = hi + x_lo_columns(LAY) * ldb;
+    const __bf16 hr = (__bf16)v.re, hm = (__bf16)v.im;
+    hi[0] = hr;
+    hi[ldb] = hm;
+    lo[0] = (__bf16)(v.re - (float)hr);
+    lo[ldb] = (__bf16)(v.im - (float)hm);
+  } else {
+    using C = cplx<typename MfmaTraits<CM>::T>;
+    reinterpret_cast<C*>(slab)[k * 8 + cf] = v;
+  }
+}
+
+// the operator's fragments of one contraction: a ring of RING chunks for the RT row tiles of a wave
+template <int CM, int RT>
+struct XRing {
+  static constexpr int RING = (CM == CM_F64 || RT >= 2) ? 2 : 4;
+  using F = typename MfmaTraits<CM>::frag_t;
+  F h[RING][RT], l[RING][CM == CM_BF16X3 ? RT : 1];
+  __device__ __forceinline__ void fetch(const F* __restrict__ hi, const F* __restrict__ lo, int nch, int m16, int mt0,
+                                        int lane, int ch, int slot) {
+    if (ch >= nch) return;
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+      if (mt0 + r < m16) {
+        const int fi = ((mt0 + r) * nch + ch) * 64 + lane;
+        h[slot][r] = hi[fi];
+        if constexpr (CM == CM_BF16X3) l[slot][r] = lo[fi];
+      }
+  }
+  __device__ __forceinline__ void start(const F* __restrict__ hi, const F* __restrict__ lo, int nch, int m16, int mt0,
+                                        int lane) {
+#pragma unroll
+    for (int d = 0; d < RING; d++) fetch(hi, lo, nch, m16, mt0, lane, d, d);
+  }
+};
+
+// acc += A . slab over all chunks (16 or 32 rows of the slab each); ring holds the first chunks' fragments. The slab
+// operands of a whole ring are read before its products.
+template <int CM, int RT, int LAY>
+__device__ __forceinline__ void x_contract(typename MfmaTraits<CM>::acc_t (&acc)[RT], XRing<CM, RT>& ring,
+                                           const typename MfmaTraits<CM>::frag_t* __restrict__ hi,
+                                           const typename MfmaTraits<CM>::frag_t* __restrict__ lo, const char* slab,
+                                           int kp, int m16, int mt0, int lane) {
+  using T = typename MfmaTraits<CM>::T;
+  constexpr int RING = XRing<CM, RT>::RING;
+  const int nch = CM == CM_BF16X3 ? kp / 32 : kp / 16;
+  const int col = lane & 15, quad = lane >> 4;
+#pragma unroll
+  for (int r = 0; r < RT; r++) acc[r] = typename MfmaTraits<CM>::acc_t{0, 0, 0, 0};
+  if (mt0 >= m16) return;  // a wave without rows
+  auto group = [&](int c0, auto whole) {
+    constexpr bool W = decltype(whole)::value;  // all RING chunks are there
+    if constexpr (CM == CM_BF16X3) {
+      constexpr bool P = LAY == X_PACK;
+      bf16x8 vh[RING], vl[P ? 1 : RING];
+      const int ldb = kp + 8;
+      const __bf16* bh = reinterpret_cast<const __bf16*>(slab) + col * ldb + c0 * 32 + 8 * quad;
+#pragma unroll
+      for (int d = 0; d < RING; d++)
+        if (W || c0 + d < nch) {
+          vh[d] = *reinterpret_cast<const bf16x8*>(bh + d * 32);
+          if constexpr (!P) vl[d] = *reinterpret_cast<const bf16x8*>(bh + d * 32 + 16 * ldb);
+        }
+#pragma unroll
+      for (int d = 0; d < RING; d++)
+        if (W || c0 + d < nch) {
+#pragma unroll
+          for (int r = 0; r < RT; r++)
+            if (mt0 + r < m16) {
+              acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring.h[d][r], vh[d], acc[r], 0, 0, 0);
+              if constexpr (!P) acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring.h[d][r], vl[d], acc[r], 0, 0, 0);
+              acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring.l[d][r], vh[d], acc[r], 0, 0, 0);
+            }
+          ring.fetch(hi, lo, nch, m16, mt0, lane, c0 + d + RING, d);
+        }
+    } else {
+      const T* bs = reinterpret_cast<const T*>(slab) + (c0 * 16 + quad) * 16 + col;
+      T b[RING][4];
+#pragma unroll
+      for (int d = 0; d < RING; d++)
+        if (W || c0 + d < nch)
+#pragma unroll
+          for (int j = 0; j < 4; j++) b[d][j] = bs[(d * 16 + 4 * j) * 16];
+#pragma unroll
+      for (int d = 0; d < RING; d++)
+        if (W || c0 + d < nch) {
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int r = 0; r < RT; r++)
+              if (mt0 + r < m16) {
+                if constexpr (CM == CM_F64)
+                  acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(ring.h[d][r][j], b[d][j], acc[r], 0, 0, 0);
+                else
+                  acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(ring.h[d][r][j], b[d][j], acc[r], 0, 0, 0);
+              }
+          ring.fetch(hi, lo, nch, m16, mt0, lane, c0 + d + RING, d);
+        }
+    }
+  };
+  int c0 = 0;
+  for (; c0 + RING <= nch; c0 += RING) group(c0, std::true_type());
+  if (c0 < nch) group(c0, std::false_type());
+}
+
+// A result tile leaves row rin(i) (i < 4) of real column lane % 16 in element i of a lane's accumulator. The two
+// lanes of a pair (one complex column) take rows i = lane % 2 + 2 p in full, p = 0 and 1; in a half-filled tile
+// (X_HALF, X_PACK) the lanes of the upper 8 columns take p = 1 for those of the lower.
+template <int CM>
+__device__ __forceinline__ int x_row_in_tile(int lane, int p) {
+  const int i = (lane & 1) + 2 * p;
+  return CM == CM_F64 ? 4 * i + (lane >> 4) : 4 * (lane >> 4) + i;
+}
+template <typename T, typename A>
+__device__ __forceinline__ cplx<T> x_pair(const A& v, int lane, int p) {
+  const T v0 = v[0], v1 = v[1], v2 = v[2], v3 = v[3];
+  const T te = p ? v2 : v0, to = p ? v3 : v1;
+  const T se = dpp_move<0xB1, 0xf>(te), so = dpp_move<0xB1, 0xf>(to);  // the pair's other lane (quad_perm 1,0,3,2)
+  return (lane & 1) ? cmk(so, to) : cmk(te, se);
+}
+// the point p of this lane (X_WIDE), or its only one
+template <int CM, int LAY>
+__device__ __forceinline__ cplx<typename MfmaTraits<CM>::T> x_point(const typename MfmaTraits<CM>::acc_t& acc,
+                                                                    int lane, int p) {
+  using T = typename MfmaTraits<CM>::T;
+  if constexpr (LAY == X_WIDE) {
+    return x_pair<T>(acc, lane, p);
+  } else {
+    typename MfmaTraits<CM>::acc_t v;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const T o = dpp_move<0x128, 0xf>((T)acc[i]);  // the lane 8 columns away (row_ror:8)
+      v[i] = LAY == X_PACK ? acc[i] + o : ((lane & 8) ? o : (T)acc[i]);
+    }
+    return x_pair<T>(v, lane, (lane >> 3) & 1);
+  }
+}
+
+// the step state's words, requested without being waited for
+struct StateWords {
+  uint4 w[sizeof(StepState) / 16];
+  __device__ __forceinline__ explicit StateWords(const StepState* st) {
+    const uint4* p = reinterpret_cast<const uint4*>(st);
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(StepState) / 16); i++) w[i] = p[i];
+  }
+  __device__ __forceinline__ StepState take() const {
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(StepState) / 16); i++)
+      asm volatile("" ::"s"(w[i].x), "s"(w[i].y), "s"(w[i].z), "s"(w[i].w));
+    StepState s;
+    __builtin_memcpy(&s, w, sizeof(StepState));
+    return s;
+  }
+};
+
+// one column tile: LAY its layout, RT its 16-row tiles per wave; LIN: a linear tile
+template <int CM, int RT, int LAY, bool LIN>
+__device__ __forceinline__ void x_tile(const XArgs<CM> a, int tile, int fc0, int hcw, char* smem, size_t slab_b) {
+  using T = typename MfmaTraits<CM>::T;
+  using C = cplx<T>;
+  using acc_t = typename MfmaTraits<CM>::acc_t;
+  __shared__ double red[16];
+  constexpr int NP = LAY == X_WIDE ? 2 : 1;  // points per lane and row tile
+  const int nth = blockDim.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwv = nth >> 6;
+  const int stage = a.stage;
+  const bool current = !LIN && stage >= 1 && stage <= 4;  // a tile that takes J
+  const long row = a.row;
+  const int mt0 = wave * RT, mk16 = (a.nk + 15) / 16, mr16 = (a.nr + 15) / 16;
+  const int nchf = CM == CM_BF16X3 ? a.kpf / 32 : a.kpf / 16, nchb = CM == CM_BF16X3 ? a.kpb / 32 : a.kpb / 16;
+  char *slab_j = smem, *slab_e = smem + slab_b;
+
+  // ---- every request of the tile up front
+  const StateWords sw(a.st);
+  __builtin_amdgcn_sched_barrier(0);
+  constexpr int JP = 2;  // pairs of rows of J in flight per thread
+  C j0[JP], j1[JP];
+  const int lgh = __builtin_ctz(hcw), npj = (a.kpf / 2) << lgh;
+  auto load_j = [&](int base) {
+#pragma unroll
+    for (int i = 0; i < JP; i++) {
+      const int e = base + tid + i * nth, k = 2 * (e >> lgh), f = fc0 + (e & (hcw - 1));
+      j0[i] = j1[i] = cmk(T(0), T(0));
+      if (e < npj && f < a.f1) {
+        if (k < a.nr) j0[i] = a.jr[k * row + f];
+        if (k + 1 < a.nr) j1[i] = a.jr[(k + 1) * row + f];
+      }
+    }
+  };
+  auto put_j = [&](int base) {
+#pragma unroll
+    for (int i = 0; i < JP; i++) {
+      const int e = base + tid + i * nth;
+      if (e < npj) x_put2<CM, LAY>(slab_j, a.kpf, 2 * (e >> lgh), e & (hcw - 1), j0[i], j1[i]);
+    }
+  };
+  if (current) load_j(0);
+  // this lane's points: row k of point p of row tile r, column f (the tile's column cl)
+  auto prow = [&](int r, int p) {
+    return (mt0 + r) * 16 + x_row_in_tile<CM>(lane, LAY == X_WIDE ? p : (lane >> 3) & 1);
+  };
+  const int cl = LAY == X_WIDE ? (lane & 15) >> 1 : (lane & 7) >> 1, f = fc0 + cl;
+  const bool col_ok = cl < hcw && f < a.nw;
+  C kz[RT][NP], Q[RT][NP], a1[RT][NP], a2[RT][NP], a3[RT][NP];
+  double ph[RT][NP];
+  const T cf = col_ok ? a.cond[f] : T(1);
+#pragma unroll
+  for (int r = 0; r < RT; r++)
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        const int k = prow(r, p);
+        kz[r][p] = cmk(T(1), T(0));
+        Q[r][p] = a1[r][p] = a2[r][p] = a3[r][p] = cmk(T(0), T(0));
+        ph[r][p] = 0.0;
+        if (k < a.nk && col_ok) {
+          const long idx = k * row + f;
+          ph[r][p] = a.phs[idx];
+          kz[r][p] = a.kzc[idx];
+          Q[r][p] = a.q[idx];
+          if (!LIN && f < a.f1) {
+            if (stage == 4 || stage == X_OPEN2) a1[r][p] = a.k1[idx];
+            if (stage == 4) {
+              a2[r][p] = a.k2[idx];
+              a3[r][p] = a.k3[idx];
+            }
+          }
+        }
+      }
+  XRing<CM, RT> ring;
+  if (current)
+    ring.start(a.fhi, a.flo, nchf, mk16, mt0, lane);
+  else
+    ring.start(a.bhi, a.blo, nchb, mr16, mt0, lane);
+
+  // ---- where this stage and the next one stand
+  const StepState st = sw.take();
+  const double dz = uniform_f64(step_dz(st));
+  const double cs = stage == 4 ? 1.0 : (stage == X_OPEN || stage == 1 ? 0.0 : 0.5);
+  const double zS = uniform_f64(st.zoff + (st.z + cs * dz));
+  constexpr bool rebased = sizeof(T) == 4;  // only FP32 states are kept relative to a reference point
+  const double qb = uniform_f64(rebased ? st.qbase : 0.0);
+  const int rb_end = __builtin_amdgcn_readfirstlane(rebased && stage == 4 && rebase_at(st, st.zoff + (st.z + dz)));
+  const int f1r = rebased ? st.rb_f1 : 0;
+  double zE = zS, cn = 0.0, qbn = qb;
+  int next = !a.est;  // whether the next stage runs
+  if (stage == 4) {
+    StepState loc = st;
+    if (loc.active) end_step(loc, dz);
+    next = loc.active && !(loc.sched_n > 0 && loc.steps >= loc.sched_n);
+    zE = loc.zoff + loc.z;
+    if (rebased) qbn = loc.qbase;
+  } else if (stage != X_OPEN) {
+    zE = st.zoff + (st.z + (stage == 3 ? 1.0 : 0.5) * dz);
+    cn = stage == 3 ? dz : dz / 2;
+  }
+  zE = uniform_f64(zE);
+  qbn = uniform_f64(qbn);
+  const T ct = (T)uniform_f64(cn);
+  if (!st.active || (st.sched_n > 0 && st.steps >= st.sched_n)) {
+    // the run has finished, or its schedule has (which the commit reports): nothing to update
+    if (!LIN && st.active && stage == 4 && tid == 0 && tile == 0 && (blockIdx.z == 0 || a.zst)) a.st->pend = 1;
+    return;
+  }
+  const bool stays = (a.keep & (stage == 2 ? 1 : (stage == 4 ? 2 : 0))) && zE == zS;
+  if (LIN && (stays || !next)) return;
+
+  // ---- Hf . J
+  acc_t acc[RT];
+  if (current) {
+    for (int base = 0;;) {
+      put_j(base);
+      base += JP * nth;
+      if (base >= npj) break;
+      load_j(base);
+    }
+    __syncthreads();
+    x_contract<CM, RT, LAY>(acc, ring, a.fhi, a.flo, slab_j, a.kpf, mk16, mt0, lane);
+    if (next) ring.start(a.bhi, a.blo, nchb, mr16, mt0, lane);
+  }
+
+  // ---- the points
+  double loc = 0.0;  // stage 1: the largest step rate Kr; stage 4: the largest |q|^2
+  bool nan = false;
+  const double amin = a.est ? st.rel_amin * bitsd(*a.qmax) : 0.0;
+  const ColRef cr{zS - qb, qb, rb_end != 0};
+#pragma unroll
+  for (int r = 0; r < RT; r++)
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        const int k = prow(r, p);
+        C J = cmk(T(0), T(0));
+        if (current) J = x_point<CM, LAY>(acc[r], lane, p);  // lanes trade parts: all of them take part
+        C v = cmk(T(0), T(0));
+        if (k < a.nk && col_ok) {
+          const long idx = k * row + f;
+          const C kzp = kz[r][p], Qp = Q[r][p];
+          const double php = ph[r][p];
+          v = Qp;
+          if (current && f < a.f1) {
+            // S = 0.5 i exp(-i(kz+kg) z) J / Re kz (uppe.cl:73-91)
+            const C t = cmul(linear_factor<T>(php, kzp.im, zS, cr.za, -1), J);
+            C S;
+            if constexpr (sizeof(T) == 4) {
+              const float rk = __builtin_amdgcn_rcpf(kzp.re);  // 1 ulp
+              S = cmk(-0.5f * t.im * rk, 0.5f * t.re * rk);
+            } else {
+              S = cmk((T(-0.5) * t.im) / kzp.re, (T(0.5) * t.re) / kzp.re);
+            }
+            if (stage == 4) {
+              const T c6 = (T)(dz / 6), c3 = (T)(dz / 3);
+              T re = Qp.re + c6 * a1[r][p].re;
+              T im = Qp.im + c6 * a1[r][p].im;
+              re = re + c3 * a2[r][p].re;
+              im = im + c3 * a2[r][p].im;
+              re = re + c3 * a3[r][p].re;
+              im = im + c3 * a3[r][p].im;
+              re = re + c6 * S.re;
+              im = im + c6 * S.im;
+              v = cmk(re * cf, im * cf);
+              const double m2 = ref_update<T>(v, kzp.im, cr, zS);
+              a.q[idx] = v;
+              loc = fmax(loc, m2);
+            } else {
+              C* ks = stage == 1 ? a.k1 : (stage == 2 ? a.k2 : a.k3);
+              ks[idx] = S;
+              if (stage == 1) {
+                const double qr = (double)Qp.re, qi = (double)Qp.im;
+                if (qr != qr || qi != qi) nan = true;  // |q| is NaN exactly when a part is
+                if (a.est) {
+                  // LoadStepSize (paraxial.cl:40-58), as in stage_point
+                  const double sr = (double)S.re, si = (double)S.im;
+                  const double am = ref_amin(amin, (double)kzp.im, cr.qb);
+                  const double rden = 1.0 / (qr * qr + qi * qi + am * am);
+                  const double alpha = (qr * sr + qi * si) * rden;
+                  const double keff = (qr * si - qi * sr) * rden;
+                  loc = fmax(loc, 0.5 * st.dphi / st.L + fabs(keff) - alpha * (double)(alpha < 0.0));
+                }
+              }
+              v = cscale(cmk(Qp.re + ct * S.re, Qp.im + ct * S.im), cf);
+            }
+          } else if (stage == X_OPEN2 && f < a.f1) {
+            v = cscale(cmk(Qp.re + ct * a1[r][p].re, Qp.im + ct * a1[r][p].im), cf);
+          } else if (stage != 4 && stage != X_OPEN) {
+            v = cscale(Qp, cf);
+          }
+          if (next) {
+            v = cmul(linear_factor<T>(php, kzp.im, zE, f < f1r ? zE - qbn : zE, +1), v);
+            if (!a.env) v = cmul(cmk(-kzp.im, kzp.re), v);  // E = i kz A
+          }
+        }
+        if (next && k < a.kpb && cl < hcw) x_put1<CM, LAY>(slab_e, a.kpb, k, cl, v);
+      }
+  if (next)  // contraction rows beyond the waves' (kpb is padded to whole chunks)
+    for (int e = tid; e < (a.kpb - nwv * RT * 16) * hcw; e += nth)
+      x_put1<CM, LAY>(slab_e, a.kpb, nwv * RT * 16 + e / hcw, e & (hcw - 1), cmk(T(0), T(0)));
+
+  // max|q| for a later adaptive step (see hankel_tile), or the smallest step estimate
+  const bool red_on = current && (a.est || (stage == 4 && !(st.fixed && st.sub + 1 < st.sub_end &&
+                                                             !(st.max_steps > 0 && st.steps + 1 >= st.max_steps))));
+  if (current && stage == 1 && nan) atomicOr(&a.st->nanflag, 1);
+  if (red_on) {
+    loc = a.est ? (loc > 0.0 ? st.dphi / loc : INFINITY) : sqrt(loc);
+    for (int o = 32; o > 0; o >>= 1) {
+      const double v = __shfl_xor(loc, o);
+      loc = a.est ? fmin(loc, v) : fmax(loc, v);
+    }
+    if (lane == 0) red[wave] = loc;
+  }
+  __syncthreads();
+  if (tid == 0 && current) {
+    if (red_on) {
+      double v = red[0];
+      for (int i = 1; i < nwv; i++) v = a.est ? fmin(v, red[i]) : fmax(v, red[i]);
+      if (a.est)
+        atomicMin(&a.st->dzraw, dbits(v));
+      else
+        atomicMax(a.qmax_next + red_slot(tile), dbits(v));
+    }
+    // the step has run; the next step's stage-1 source launch commits its end
+    if (stage == 4 && tile == 0 && (blockIdx.z == 0 || a.zst)) a.st->pend = 1;
+  }
+  if (!next) return;
+
+  // ---- Hb . E
+  x_contract<CM, RT, LAY>(acc, ring, a.bhi, a.blo, slab_e, a.kpb, mr16, mt0, lane);
+#pragma unroll
+  for (int r = 0; r < RT; r++)
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        const C v = x_point<CM, LAY>(acc[r], lane, p);
+        const int k = prow(r, p);
+        if (k < a.nr && col_ok) a.er[k * row + f] = v;
+      }
+}
+
+// LAY: the nl tiles' layout; RT: 16-row tiles per wave. Linear tiles are X_WIDE ones.
+template <int CM, int RT, int LAY>
+__global__ __launch_bounds__(64 * x_max_waves(CM)) void f_exchange(XArgs<CM> a) {
+  extern __shared__ __align__(16) char smem[];
+  const int b = blockIdx.x;
+  if (a.zs) {
+    // instance blockIdx.z of a batched launch (or azimuthal mode): see hankel_tile
+    const long z = blockIdx.z, zo = z * a.zs;
+    const long sf = (long)((a.nk + 15) / 16) * (CM == CM_BF16X3 ? a.kpf / 32 : a.kpf / 16) * 64;
+    const long sb = (long)((a.nr + 15) / 16) * (CM == CM_BF16X3 ? a.kpb / 32 : a.kpb / 16) * 64;
+    if (!(a.share & 1)) {
+      a.fhi += z * sf;
+      a.bhi += z * sb;
+      if constexpr (CM == CM_BF16X3) {
+        a.flo += z * sf;
+        a.blo += z * sb;
+      }
+    }
+    if (!(a.share & 2)) {
+      a.phs += zo;
+      a.kzc += zo;
+    }
+    a.jr += zo;
+    a.er += zo;
+    a.q += zo;
+    a.k1 += zo;
+    a.k2 += zo;
+    a.k3 += zo;
+    if (a.zst) {
+      a.st += z;
+      a.qmax += (long)kQW * z;
+      a.qmax_next += (long)kQW * z;
+    }
+  }
+  const size_t slab_b = max(x_slab_bytes<CM>(a.kpf), x_slab_bytes<CM>(a.kpb));
+  if (b < a.nlt) {
+    const int tile = xcd_tile(b, a.nlt);
+    x_tile<CM, RT, LAY, false>(a, tile, tile * a.wn, a.wn, smem, slab_b);
+  } else {
+    const int tile = xcd_tile(b - a.nlt, (int)gridDim.x - a.nlt);
+    x_tile<CM, RT, X_WIDE, true>(a, tile, a.nlt * a.wn + tile * a.wl, a.wl, smem, slab_b);
+  }
+}
+
 // ---------------------------------------------------------------------------------------------------
 // Cartesian transverse transforms (grid_tools.py:218-250; FFT_axis1/2, IFFT_axis1/2: fft.cl:387-441)
 //
@@ -1582,20 +2136,6 @@ __device__ inline void lds_write_reals(cplx<T>* Y, int n0, const T* src) {
   } else {
 #pragma unroll
     for (int j = 0; j < RUN; j++) lds_sample(Y, n0 + j) = src[j];
-  }
-}
-
-// DPP lane move (gfx9 control codes: row_shr:n = 0x110 + n, wave_shr:1 = 0x138, row_bcast:15 = 0x142,
-// row_bcast:31 = 0x143); lanes without a source, or in rows outside RM, read 0
-template <int CTRL, int RM, typename T>
-__device__ inline T dpp_move(T v) {
-  if constexpr (sizeof(T) == 4) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, RM, 0xf, false));
-  } else {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, RM, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, RM, 0xf, false);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
   }
 }
 
@@ -3000,6 +3540,44 @@ static int hk_chunk(int cm, int kp, int bm, int bn) {
   return kch;
 }
 
+// dynamic LDS of one exchange workgroup: the B slabs of both contractions
+static size_t x_lds(int cm, int kpf, int kpb) {
+  const int kp = std::max(kpf, kpb);
+  return 2 * (cm == CM_F64 ? x_slab_bytes<CM_F64>(kp) : (cm == CM_F32 ? x_slab_bytes<CM_F32>(kp) : x_slab_bytes<CM_BF16X3>(kp)));
+}
+
+// exchange over nr radial cells in nl tiles of wn complex columns (4 or 8); wn = 0 in the result where no kernel
+// has the shape: wide tiles with more than 2 row tiles per wave in FP64, or more than one elsewhere, would spill
+static FusedState::XPlan x_shape(int cm, int nr, int wn) {
+  FusedState::XPlan p;
+  const int m16 = (nr + 15) / 16;
+  p.nwv = std::min(x_max_waves(cm), m16);
+  p.rt = (m16 + p.nwv - 1) / p.nwv;
+  if (p.rt == 3) p.rt = 4;
+  p.wl = 8;
+  p.wn = p.rt > (cm == CM_F64 ? 4 : 2) || (wn > 4 && p.rt > (cm == CM_F64 ? 2 : 1)) ? 0 : wn;
+  return p;
+}
+
+// The exchange plan of one grid (wn = 0: separate contractions). Tiles of 4 complex columns put a grid's points on
+// twice the CUs that tiles of 8 do, as long as all tiles (the nl ones, and the linear ones of 8) run at once; past
+// that the operator, which every tile reads whole, is the larger cost. Measured, us per step, separate / 4 / 8
+// columns: BF16x3 Kerr 513 x 128 66 / 50 / 55, O2 2049 x 256 117 / 111 / 106; FP64 513 x 128 109 / 77 / 81,
+// O2 1025 x 128 201 / 173 / 169. Above 256 cells one tile's contractions hold a CU for longer than the separate
+// kernels, which split their rows over CUs, unless the grid has tiles for every CU (BF16x3 513 x 512 123 / 117;
+// FP64 2049 x 512 1486 / 680, 513 x 512 298 / 363); FP32 stays with them (513 x 512 194 / 230).
+static FusedState::XPlan plan_exchange(int cm, int nr, int f1, int nw, int instances, int n_cu) {
+  // SEARAY_UPPE_TILE_WIDTH pins the tiling of the separate contractions, so it asks for them
+  if (cm < 0 || nr > 512 || getenv("SEARAY_UPPE_TILE_WIDTH")) return FusedState::XPlan();
+  const int nlt = (f1 + 3) / 4, lin = (std::max(0, nw - 4 * nlt) + 7) / 8;
+  const bool at_once = (long)(nlt + lin) * instances <= n_cu;
+  if (nr > 256) {
+    if (cm == CM_F32 || at_once != (cm == CM_BF16X3)) return FusedState::XPlan();
+    return x_shape(cm, nr, 4);
+  }
+  return x_shape(cm, nr, at_once ? 4 : 8);
+}
+
 template <typename T>
 void tune_single(uppe_handle* h, FusedState* s, bool may_time = true);
 
@@ -3222,6 +3800,7 @@ struct Fused {
     }
     s->plan[0] = plan_hankel(nr, h->nw, s->n_cu);
     s->plan[1] = plan_hankel(nk, s->f1, s->n_cu);
+    s->xplan = plan_exchange(s->cm, nr, s->f1, h->nw, h->n2, s->n_cu);
     s->tuned_f1 = -1;
   }
 
@@ -3262,10 +3841,15 @@ struct Fused {
     // columns at and above f1 carry zero current: the r2k contraction and the stage updates skip them.
     // f1 covers the conditioner's four bins.
     const int f1 = std::min(h->nw, std::max(last_nl + 1, 4));
+    s->cond_one = true;
+    for (int f = f1; f < h->nw; f++) s->cond_one = s->cond_one && m->cond_filter[f] == 1.0;
     if (moved) end_medium_change(h, s, f1);
     if (f1 != s->f1) {
       s->f1 = f1;
-      if (h->have_hankel) s->plan[1] = plan_hankel(h->nk, s->f1, s->n_cu);
+      if (h->have_hankel) {
+        s->plan[1] = plan_hankel(h->nk, s->f1, s->n_cu);
+        s->xplan = plan_exchange(s->cm, h->n1, s->f1, h->nw, h->n2, s->n_cu);
+      }
       const size_t cs = sizeof(C) * P * s->nwp;
       UPPE_HIP(hipMemset(s->k1, 0, cs));
       UPPE_HIP(hipMemset(s->k2, 0, cs));
@@ -3302,10 +3886,14 @@ struct Fused {
     s->ion = m->ion;
     s->max_ki = 0.0;
     for (long i = 0; i < h->npt; i++) s->max_ki = std::max(s->max_ki, m->kz[2 * i + 1]);
+    s->cond_one = true;
     if (moved) end_medium_change(h, s, h->nw);
     if (h->nw != s->f1) {
       s->f1 = h->nw;
-      if (h->have_hankel) s->plan[1] = plan_hankel(h->nk, s->f1, s->n_cu);
+      if (h->have_hankel) {
+        s->plan[1] = plan_hankel(h->nk, s->f1, s->n_cu);
+        s->xplan = plan_exchange(s->cm, h->n1, s->f1, h->nw, h->n2, s->n_cu);
+      }
       const size_t cs = sizeof(C) * P * s->nwp;
       UPPE_HIP(hipMemset(s->k1, 0, cs));
       UPPE_HIP(hipMemset(s->k2, 0, cs));
@@ -3563,21 +4151,122 @@ struct Fused {
                             stage, zfix, 0.0, 0.0);
   }
 
-  // one RK4 step; with erslot, stage s leaves its E_r in erslot[s - 1] (slots of P nwp points) for the adjoint
+  // one exchange launch: J_r (jr) to the slope and state of `stage` and on to the next stage's E_r (er). keep: see
+  // XArgs
   template <int CM>
-  static void step_mfma(uppe_handle* h, FusedState* s, C* erslot = nullptr) {
-    const C* kp[5] = {nullptr, nullptr, (const C*)s->k1, (const C*)s->k2, (const C*)s->k3};
-    const long stride = h->P * (long)s->nwp;
-    for (int stage = 1; stage <= 4; stage++) {
-      C* er = erslot ? erslot + (stage - 1) * stride : (C*)s->er;
-      if (h->paraxial)
-        hankel_mfma<CM, PRO_STAGE_ENV, EPI_NONE>(h, s, 0, (const C*)s->q, er, kp[stage], stage, 0.0, s->st);
+  static void x_launch(uppe_handle* h, FusedState* s, const FusedState::XPlan& pl, const C* jr, C* er, int stage,
+                       bool est, int keep, int nz = 1, long zs = 0, int share = 0) {
+    using F = typename MfmaTraits<CM>::frag_t;
+    int zst = 1;
+    long row = s->nwp;
+    if (zs == 0 && h->n2 > 1) {  // azimuthal modes: see hk_launch
+      nz = h->n2;
+      zs = s->nwp;
+      zst = 0;
+      row = (long)h->n2 * s->nwp;
+    }
+    XArgs<CM> a;
+    a.fhi = (const F*)s->frf_hi;
+    a.flo = (const F*)s->frf_lo;
+    a.bhi = (const F*)s->frb_hi;
+    a.blo = (const F*)s->frb_lo;
+    a.jr = jr;
+    a.er = er;
+    a.phs = s->phs;
+    a.kzc = (const C*)s->kzc;
+    a.cond = (const T*)s->cond;
+    a.q = (C*)s->q;
+    a.k1 = (C*)s->k1;
+    a.k2 = (C*)s->k2;
+    a.k3 = (C*)s->k3;
+    a.st = s->st;
+    a.qmax = s->qmax;
+    a.qmax_next = s->qmax_next;
+    a.zs = zs;
+    a.nr = h->n1;
+    a.nk = h->nk;
+    a.kpf = s->kp_f;
+    a.kpb = s->kp_b;
+    a.row = (int)row;
+    a.f1 = s->f1;
+    a.nw = h->nw;
+    a.wn = pl.wn;
+    a.wl = pl.wl;
+    a.nlt = (s->f1 + pl.wn - 1) / pl.wn;
+    a.stage = stage;
+    a.est = est ? 1 : 0;
+    a.env = h->paraxial ? 1 : 0;
+    a.zst = zst;
+    a.share = zst ? share : 0;
+    a.keep = keep;
+    const int lin = std::max(0, (h->nw - a.nlt * pl.wn + pl.wl - 1) / pl.wl);
+    const size_t shm = x_lds(CM, a.kpf, a.kpb);
+    if (pl.wn < 1 || 16 * pl.nwv * pl.rt < h->n1 || shm > kMaxLds)
+      throw Error{UPPE_ERR_STATE, "exchange plan out of date"};
+    // no linear tile has anything to do from stage 2 to 3, where the phase coordinate stands still, and in a launch
+    // that ends with its slopes
+    const dim3 grid((unsigned)(a.nlt + (est || ((keep & 1) && stage == 2) ? 0 : lin)), 1, (unsigned)nz);
+#define UPPE_X(RTV, LAY)                                                                                          \
+  launchf(h, UPPE_KC_EXCHANGE, f_exchange<CM, RTV, LAY>, grid, dim3(64 * pl.nwv), shm, a)
+    constexpr int half = CM == CM_BF16X3 ? X_PACK : X_HALF;
+    const bool wide = pl.wn > 4;
+    if (pl.rt == 1) {
+      if (wide)
+        UPPE_X(1, X_WIDE);
       else
-        hankel_mfma<CM, PRO_STAGE, EPI_NONE>(h, s, 0, (const C*)s->q, er, kp[stage], stage, 0.0, s->st);
+        UPPE_X(1, half);
+    } else if (pl.rt == 2 && !wide) {
+      UPPE_X(2, half);
+    } else if constexpr (CM == CM_F64) {  // the shapes x_shape admits
+      if (wide)
+        UPPE_X(2, X_WIDE);
+      else
+        UPPE_X(4, half);
+    }
+#undef UPPE_X
+  }
+
+  // the k2r contraction of `stage` with its stage prologue
+  template <int CM>
+  static void k2r_stage(uppe_handle* h, FusedState* s, C* er, int stage) {
+    const C* kp[5] = {nullptr, nullptr, (const C*)s->k1, (const C*)s->k2, (const C*)s->k3};
+    if (h->paraxial)
+      hankel_mfma<CM, PRO_STAGE_ENV, EPI_NONE>(h, s, 0, (const C*)s->q, er, kp[stage], stage, 0.0, s->st);
+    else
+      hankel_mfma<CM, PRO_STAGE, EPI_NONE>(h, s, 0, (const C*)s->q, er, kp[stage], stage, 0.0, s->st);
+  }
+
+  // One RK4 step of a run that opened with `first`: its stage-1 E_r comes from a k2r launch on the first step and
+  // from the step before on the others. known: the step size does not depend on stage 1's slope (fixed and
+  // replayed steps). With erslot, stage s leaves its E_r in erslot[s - 1] (slots of P nwp points) for the adjoint;
+  // er_next receives the next step's.
+  template <int CM>
+  static void step_mfma(uppe_handle* h, FusedState* s, bool first, bool known, C* erslot = nullptr,
+                        C* er_next = nullptr) {
+    const long stride = h->P * (long)s->nwp;
+    const bool x = s->xplan.wn > 0;
+    auto slot = [&](int stage) {
+      if (!erslot) return (C*)s->er;
+      return stage <= 4 ? erslot + (stage - 1) * stride : (er_next ? er_next : (C*)s->er);
+    };
+    const int keep = (!erslot && h->n2 == 1) ? 1 | (s->cond_one ? 2 : 0) : 0;
+    if (!x)
+      k2r_stage<CM>(h, s, slot(1), 1);
+    else if (first)
+      x_launch<CM>(h, s, s->xplan, (const C*)s->jr, slot(1), X_OPEN, false, 0);
+    for (int stage = 1; stage <= 4; stage++) {
+      C* er = slot(stage);
       azim(h, s, er, h->nw, +1);  // azimuthal modes to phi (IFFT_axis2 after the radial transform)
       source(h, s, (const C*)er, (C*)s->jr, false, stage == 1 ? s->st : nullptr, 1, nullptr, 0, s->spt);
       azim(h, s, (C*)s->jr, s->f1, -1);  // phi to modes over the nonlinear band (FFT_axis2 first)
-      hankel_mfma<CM, PRO_NONE, EPI_STAGE>(h, s, 1, (const C*)s->jr, (C*)nullptr, nullptr, stage, 0.0, s->st);
+      if (x) {
+        const bool est = stage == 1 && !known;
+        x_launch<CM>(h, s, s->xplan, (const C*)s->jr, slot(stage + 1), stage, est, keep);
+        if (est) x_launch<CM>(h, s, s->xplan, (const C*)s->jr, slot(2), X_OPEN2, false, keep);
+      } else {
+        hankel_mfma<CM, PRO_NONE, EPI_STAGE>(h, s, 1, (const C*)s->jr, (C*)nullptr, nullptr, stage, 0.0, s->st);
+        if (stage < 4) k2r_stage<CM>(h, s, slot(stage + 1), stage + 1);
+      }
     }
   }
 
@@ -3631,19 +4320,19 @@ struct Fused {
     }
   }
 
-  static void step(uppe_handle* h, FusedState* s) {
+  static void step(uppe_handle* h, FusedState* s, bool first, bool known) {
     if (h->d.geometry == UPPE_CARTESIAN) {
       step_cart(h, s);
       return;
     }
     if (s->cm >= 0) {
       if constexpr (sizeof(T) == 8) {
-        step_mfma<CM_F64>(h, s);
+        step_mfma<CM_F64>(h, s, first, known);
       } else {
         if (s->cm == CM_BF16X3)
-          step_mfma<CM_BF16X3>(h, s);
+          step_mfma<CM_BF16X3>(h, s, first, known);
         else
-          step_mfma<CM_F32>(h, s);
+          step_mfma<CM_F32>(h, s, first, known);
       }
       return;
     }
@@ -3792,6 +4481,7 @@ struct Fused {
       s->er_cap = 4 * every;
     }
     s->recorded = false;
+    const bool known = sh->fixed || sh->sched_n > 0;
     int seg = 0;
     while (true) {
       grow(&s->zrec, &s->zrec_cap, 3 * (seg + 1) * every, sizeof(double), h->stream);
@@ -3803,7 +4493,10 @@ struct Fused {
       UPPE_HIP(hipMemcpyAsync(s->ck_qmax + (long)kQW * seg, s->qmax, kQW * sizeof(unsigned long long), hipMemcpyDeviceToDevice,
                               h->stream));
       s->zrec_active = s->zrec;
-      for (int i = 0; i < every; i++) step_mfma<CM>(h, s, (C*)s->er_store + (long)i * 4 * stride);
+      // (the segment's last step leaves the next segment's first E_r in the first slot; the run's last leaves none)
+      for (int i = 0; i < every; i++)
+        step_mfma<CM>(h, s, seg == 0 && i == 0, known, (C*)s->er_store + (long)i * 4 * stride,
+                      (C*)s->er_store + (long)((i + 1) % every) * 4 * stride);
       commit(h, s);
       s->zrec_active = nullptr;
       UPPE_HIP(hipMemcpyAsync(sh, s->st, sizeof(StepState), hipMemcpyDeviceToHost, h->stream));
@@ -3817,6 +4510,7 @@ struct Fused {
     s->ck_every = every;
     s->ck_n = (steps + every - 1) / every;
     s->rec_steps = steps;
+    s->rec_known = known;
     s->zrec_host.resize((size_t)3 * steps);
     if (steps > 0)
       UPPE_HIP(hipMemcpy(s->zrec_host.data(), s->zrec, sizeof(double) * 3 * steps, hipMemcpyDeviceToHost));
@@ -3867,7 +4561,9 @@ struct Fused {
                                 hipMemcpyDeviceToDevice, h->stream));
         s->rec_active = nullptr;
         s->zrec_active = nullptr;
-        for (int i = 0; i < n1 - n0; i++) step_mfma<CM>(h, s, (C*)s->er_store + (long)i * 4 * stride);
+        for (int i = 0; i < n1 - n0; i++)
+          step_mfma<CM>(h, s, i == 0, s->rec_known, (C*)s->er_store + (long)i * 4 * stride,
+                        i + 1 < n1 - n0 ? (C*)s->er_store + (long)(i + 1) * 4 * stride : nullptr);
       }
       for (int n = n1 - 1; n >= n0; n--) {
         const double zoff = zr[3 * n], z = zr[3 * n + 1], dz = zr[3 * n + 2];
@@ -3996,10 +4692,11 @@ struct Fused {
     UPPE_HIP(hipMemcpyAsync(s->st, sh, sizeof(StepState), hipMemcpyHostToDevice, h->stream));
     tune_single<T>(h, s, may_time);
     long long guard = 0;
+    const bool known = sh->fixed || sh->sched_n > 0;
     int chunk = c->n_sub;
     if (sh->max_steps > 0) chunk = std::min(chunk, sh->max_steps);
     while (true) {
-      for (int i = 0; i < chunk; i++) step(h, s);
+      for (int i = 0; i < chunk; i++) step(h, s, guard == 0 && i == 0, known);
       commit(h, s);
       UPPE_HIP(hipMemcpyAsync(sh, s->st, sizeof(StepState), hipMemcpyDeviceToHost, h->stream));
       UPPE_HIP(hipStreamSynchronize(h->stream));
@@ -4104,6 +4801,8 @@ struct BatchRun {
   int group = 0, first = 0, count = 0;  // slots [first, first + count) of the group
   FusedState::HkPlan plan[2];           // k2r, r2k
   int spt = 0;                          // source samples per thread (0: the single-instance choice)
+  FusedState::XPlan xplan;              // exchange (wn = 0: none)
+  bool known = false;                   // no member's step size depends on its stage 1 (fixed steps)
   int share = 0;  // bit 0: the members' operators agree, bit 1: their kz tables agree (one copy is read)
 };
 
@@ -4236,8 +4935,17 @@ void fused_batch_plan(const uppe_batch* b, int member, int* out) {
   const int g = fb->group_of[(size_t)member], j = fb->slot_of[(size_t)member];
   for (const BatchRun& r : fb->runs) {
     if (r.group != g || j < r.first || j >= r.first + r.count) continue;
-    const int v[10] = {r.plan[0].tiles, r.plan[0].nwv, r.plan[0].rt, r.plan[1].tiles, r.plan[1].nwv,
-                       r.plan[1].rt,    r.spt,         r.count,      r.first,         g};
+    int v[10] = {r.plan[0].tiles, r.plan[0].nwv, r.plan[0].rt, r.plan[1].tiles, r.plan[1].nwv,
+                 r.plan[1].rt,    r.spt,         r.count,      r.first,         g};
+    if (r.xplan.wn > 0) {
+      // exchanges take both directions: all their tiles, and those of the nonlinear band
+      const uppe_handle* h = b->members[(size_t)member];
+      const int nlt = (h->fused->f1 + r.xplan.wn - 1) / r.xplan.wn;
+      v[0] = nlt + std::max(0, (h->nw - nlt * r.xplan.wn + r.xplan.wl - 1) / r.xplan.wl);
+      v[3] = nlt;
+      v[1] = v[4] = r.xplan.nwv;
+      v[2] = v[5] = r.xplan.rt;
+    }
     std::memcpy(out, v, sizeof(v));
     return;
   }
@@ -4249,24 +4957,67 @@ struct BatchOps {
   using F = Fused<T>;
   using C = cplx<T>;
 
-  // one RK4 step of a run: step_mfma with every launch covering the run's instances
+  // the k2r contraction of `stage` over the run's instances
+  template <int CM>
+  static void k2r_run(uppe_batch* b, const BatchRun& r, int stage) {
+    const BatchGroup& G = b->fb->groups[(size_t)r.group];
+    uppe_handle* h = b->members[(size_t)G.members[(size_t)r.first]];
+    FusedState* s = h->fused;
+    const C* kp[5] = {nullptr, nullptr, (const C*)s->k1, (const C*)s->k2, (const C*)s->k3};
+    F::template hk_launch<CM, PRO_STAGE, EPI_NONE>(h, s, s->frb_hi, s->frb_lo, s->kp_b, h->n1, h->nk, h->nw, r.plan[0],
+                                                   (const C*)s->q, (C*)s->er, kp[stage], (C*)s->q, (C*)s->k1, (C*)s->k2,
+                                                   (C*)s->k3, s->st, stage, 0.0, 0.0, 0.0, r.count,
+                                                   h->P * (long)s->nwp, r.share);
+  }
+
+  // one RK4 step of a run: step_mfma with every launch covering the run's instances. Where the run takes exchanges,
+  // the first step's E_r is there already (start_run).
   template <int CM>
   static void step_run(uppe_batch* b, const BatchRun& r) {
     const BatchGroup& G = b->fb->groups[(size_t)r.group];
     uppe_handle* h = b->members[(size_t)G.members[(size_t)r.first]];
     FusedState* s = h->fused;
     const long zs = h->P * (long)s->nwp;
-    const C* kp[5] = {nullptr, nullptr, (const C*)s->k1, (const C*)s->k2, (const C*)s->k3};
     C *q = (C*)s->q, *k1 = (C*)s->k1, *k2 = (C*)s->k2, *k3 = (C*)s->k3;
+    const bool x = r.xplan.wn > 0;
+    if (!x) k2r_run<CM>(b, r, 1);
     for (int stage = 1; stage <= 4; stage++) {
-      F::template hk_launch<CM, PRO_STAGE, EPI_NONE>(h, s, s->frb_hi, s->frb_lo, s->kp_b, h->n1, h->nk, h->nw,
-                                                     r.plan[0], (const C*)q, (C*)s->er, kp[stage], q, k1, k2, k3,
-                                                     s->st, stage, 0.0, 0.0, 0.0, r.count, zs, r.share);
       F::source(h, s, (const C*)s->er, (C*)s->jr, false, stage == 1 ? s->st : nullptr, r.count, G.src + r.first, zs,
                 r.spt);
-      F::template hk_launch<CM, PRO_NONE, EPI_STAGE>(h, s, s->frf_hi, s->frf_lo, s->kp_f, h->nk, h->n1, s->f1,
-                                                     r.plan[1], (const C*)s->jr, (C*)nullptr, nullptr, q, k1, k2,
-                                                     k3, s->st, stage, 0.0, 0.0, 0.0, r.count, zs, r.share);
+      if (x) {
+        const int keep = 1 | (s->cond_one ? 2 : 0);
+        const bool est = stage == 1 && !r.known;
+        F::template x_launch<CM>(h, s, r.xplan, (const C*)s->jr, (C*)s->er, stage, est, keep, r.count, zs, r.share);
+        if (est)
+          F::template x_launch<CM>(h, s, r.xplan, (const C*)s->jr, (C*)s->er, X_OPEN2, false, keep, r.count, zs,
+                                   r.share);
+      } else {
+        F::template hk_launch<CM, PRO_NONE, EPI_STAGE>(h, s, s->frf_hi, s->frf_lo, s->kp_f, h->nk, h->n1, s->f1,
+                                                       r.plan[1], (const C*)s->jr, (C*)nullptr, nullptr, q, k1, k2,
+                                                       k3, s->st, stage, 0.0, 0.0, 0.0, r.count, zs, r.share);
+        if (stage < 4) k2r_run<CM>(b, r, stage + 1);
+      }
+    }
+  }
+
+  // the stage-1 E_r of a run's first step, where its steps take exchanges
+  static void start_run(uppe_batch* b, const BatchRun& r) {
+    if (r.xplan.wn == 0) return;
+    const BatchGroup& G = b->fb->groups[(size_t)r.group];
+    uppe_handle* h = b->members[(size_t)G.members[(size_t)r.first]];
+    FusedState* s = h->fused;
+    const long zs = h->P * (long)s->nwp;
+    auto open = [&](auto cm) {
+      F::template x_launch<decltype(cm)::value>(h, s, r.xplan, (const C*)s->jr, (C*)s->er, X_OPEN, false, 0, r.count, zs,
+                                                r.share);
+    };
+    if constexpr (sizeof(T) == 8) {
+      open(std::integral_constant<int, CM_F64>());
+    } else {
+      if (G.cm == CM_BF16X3)
+        open(std::integral_constant<int, CM_BF16X3>());
+      else
+        open(std::integral_constant<int, CM_F32>());
     }
   }
 
@@ -4336,7 +5087,8 @@ struct BatchOps {
   // when it is 3 % faster, so that timing noise does not pick between equals.
   template <int CM>
   static void tune_shapes(uppe_handle* h, FusedState* s, int nz, long zs, const SrcInst* src,
-                          FusedState::HkPlan plan[2], int* spt_out, int share = 0) {
+                          FusedState::HkPlan plan[2], FusedState::XPlan* xplan, int* spt_out,
+                          int share = 0) {
     C *q = (C*)s->q, *k1 = (C*)s->k1, *k2 = (C*)s->k2, *k3 = (C*)s->k3;
     hipEvent_t e0, e1;
     UPPE_HIP(hipEventCreate(&e0));
@@ -4363,22 +5115,45 @@ struct BatchOps {
                                                          2, 0.0, 0.0, 0.0, nz, zs, share);
         }, reps);
       };
-      // with the tile width pinned, the default plan is not a candidate: the first candidate is taken
-      const bool pinned = getenv("SEARAY_UPPE_TILE_WIDTH") != nullptr;
-      float best = pinned ? 1e30f : k2r(plan[0]);
-      for (const auto& p : candidates(s->cm, h->n1, h->nw, s->kp_b)) {
-        const float t = k2r(p);
-        if (t < margin * best) {
-          best = t;
-          plan[0] = p;
+      // exchanges at a stage whose linear tiles run (3) and one whose do not (2)
+      float best = 0.f;
+      if (xplan && xplan->wn > 0) {
+        auto xch = [&](const FusedState::XPlan& p) {
+          return time_launch(h->stream, e0, e1, [&] {
+            F::template x_launch<CM>(h, s, p, (const C*)s->jr, (C*)s->er, 2, false, 1, nz, zs, share);
+            F::template x_launch<CM>(h, s, p, (const C*)s->jr, (C*)s->er, 3, false, 1, nz, zs, share);
+          }, reps);
+        };
+        best = xch(*xplan);
+        for (int w = 4; w <= 8; w *= 2) {
+          const FusedState::XPlan p = x_shape(s->cm, h->n1, w);
+          if (p.wn == 0) continue;
+          const float t = xch(p);
+          if (t < margin * best) {
+            best = t;
+            *xplan = p;
+          }
         }
       }
-      best = pinned ? 1e30f : r2k(plan[1]);
-      for (const auto& p : candidates(s->cm, h->nk, s->f1, s->kp_f)) {
-        const float t = r2k(p);
-        if (t < margin * best) {
-          best = t;
-          plan[1] = p;
+      // the separate contractions, where the steps take them
+      if (!(xplan && xplan->wn > 0)) {
+        // with the tile width pinned, the default plan is not a candidate: the first candidate is taken
+        const bool pinned = getenv("SEARAY_UPPE_TILE_WIDTH") != nullptr;
+        best = pinned ? 1e30f : k2r(plan[0]);
+        for (const auto& p : candidates(s->cm, h->n1, h->nw, s->kp_b)) {
+          const float t = k2r(p);
+          if (t < margin * best) {
+            best = t;
+            plan[0] = p;
+          }
+        }
+        best = pinned ? 1e30f : r2k(plan[1]);
+        for (const auto& p : candidates(s->cm, h->nk, s->f1, s->kp_f)) {
+          const float t = r2k(p);
+          if (t < margin * best) {
+            best = t;
+            plan[1] = p;
+          }
         }
       }
       if (src && !getenv("SEARAY_UPPE_SOURCE_SPT") && h->rot_states <= 2) {  // a pinned shape is kept, and the
@@ -4412,14 +5187,15 @@ struct BatchOps {
   }
 
   static void tune_shapes(uppe_handle* h, FusedState* s, int nz, long zs, const SrcInst* src,
-                          FusedState::HkPlan plan[2], int* spt_out, int share = 0) {
+                          FusedState::HkPlan plan[2], FusedState::XPlan* xplan, int* spt_out,
+                          int share = 0) {
     if constexpr (sizeof(T) == 8) {
-      tune_shapes<CM_F64>(h, s, nz, zs, src, plan, spt_out, share);
+      tune_shapes<CM_F64>(h, s, nz, zs, src, plan, xplan, spt_out, share);
     } else {
       if (s->cm == CM_BF16X3)
-        tune_shapes<CM_BF16X3>(h, s, nz, zs, src, plan, spt_out, share);
+        tune_shapes<CM_BF16X3>(h, s, nz, zs, src, plan, xplan, spt_out, share);
       else
-        tune_shapes<CM_F32>(h, s, nz, zs, src, plan, spt_out, share);
+        tune_shapes<CM_F32>(h, s, nz, zs, src, plan, xplan, spt_out, share);
     }
   }
 
@@ -4427,7 +5203,7 @@ struct BatchOps {
   static void tune(uppe_batch* b, BatchRun& r) {
     const BatchGroup& G = b->fb->groups[(size_t)r.group];
     uppe_handle* h = b->members[(size_t)G.members[(size_t)r.first]];
-    tune_shapes(h, h->fused, r.count, h->P * (long)h->fused->nwp, G.src + r.first, r.plan, &r.spt, r.share);
+    tune_shapes(h, h->fused, r.count, h->P * (long)h->fused->nwp, G.src + r.first, r.plan, &r.xplan, &r.spt, r.share);
   }
 };
 
@@ -4459,7 +5235,7 @@ void tune_single(uppe_handle* h, FusedState* s, bool may_time) {
   const char* env = getenv("SEARAY_UPPE_TUNE");
   if (env && env[0] == '1') {
     int unused = 0;
-    BatchOps<T>::tune_shapes(h, s, 1, 0, nullptr, s->plan, &unused);
+    BatchOps<T>::tune_shapes(h, s, 1, 0, nullptr, s->plan, nullptr, &unused);
   }
   s->spt = default_spt(h, s, h->P);
   s->tuned_f1 = s->f1;
@@ -4568,6 +5344,9 @@ void fused_batch_advance(uppe_batch* b, const uppe_step_control* c, int* steps_o
       r.count = j - r.first;
       r.plan[0] = h0->fused->plan[0];
       r.plan[1] = h0->fused->plan[1];
+      r.xplan = h0->fused->xplan;
+      r.known = true;
+      for (int m = r.first; m < r.first + r.count; m++) r.known = r.known && G.st_host[m].fixed;
       r.spt = default_spt(h0, h0->fused, (long)r.count * h0->P);
       // members whose operators (or kz tables) have equal fingerprints read the first member's copy: one copy
       // stays in the caches where the run's instances would each stream their own
@@ -4581,7 +5360,9 @@ void fused_batch_advance(uppe_batch* b, const uppe_step_control* c, int* steps_o
         const std::vector<long> key = {g, r.first, r.count, h0->fused->f1, r.share};
         auto it = std::find_if(fb->tuned.begin(), fb->tuned.end(), [&](const auto& e) { return e.first == key; });
         if (it != fb->tuned.end()) {
+          const bool known = r.known;
           r = it->second;
+          r.known = known;
         } else {
           if (G.prec == UPPE_PREC_FP64)
             BatchOps<double>::tune(b, r);
@@ -4607,7 +5388,17 @@ void fused_batch_advance(uppe_batch* b, const uppe_step_control* c, int* steps_o
   bool prof = false;
   for (const uppe_handle* h : b->members) prof = prof || h->prof;
   const int gs = prof ? 0 : fb->graph_steps;
-  if (gs > 0) build_graph(b, gs);
+  for (const BatchRun& r : fb->runs) {
+    if (fb->groups[(size_t)r.group].prec == UPPE_PREC_FP64)
+      BatchOps<double>::start_run(b, r);
+    else
+      BatchOps<float>::start_run(b, r);
+  }
+  if (gs > 0) {
+    build_graph(b, gs);
+    // the graph runs on a stream of its own
+    for (const BatchRun& r : fb->runs) UPPE_HIP(hipStreamSynchronize(run_stream(b, r)));
+  }
   long long guard = 0;
   while (true) {
     int ran = 0;
