@@ -1453,6 +1453,108 @@ struct StateWords {
   }
 };
 
+// where an exchange of `stage` stands: the step size, the phase coordinates of this stage (zS) and the next (zE), the
+// next stage's RK coefficient, the reference point of the rebased columns now and for the next stage, whether this
+// step's update moves it, and whether the next stage runs
+struct XPos {
+  double dz, zS, zE, qb, qbn;
+  double cn;
+  int rb_end, f1r, next;
+};
+template <typename T>
+__device__ __forceinline__ XPos x_pos(const StepState& st, int stage, bool est) {
+  constexpr bool rebased = sizeof(T) == 4;  // only FP32 states are kept relative to a reference point
+  XPos x;
+  x.dz = uniform_f64(step_dz(st));
+  const double cs = stage == 4 ? 1.0 : (stage == X_OPEN || stage == 1 ? 0.0 : 0.5);
+  x.zS = uniform_f64(st.zoff + (st.z + cs * x.dz));
+  x.qb = uniform_f64(rebased ? st.qbase : 0.0);
+  x.rb_end = __builtin_amdgcn_readfirstlane(rebased && stage == 4 && rebase_at(st, st.zoff + (st.z + x.dz)));
+  x.f1r = rebased ? st.rb_f1 : 0;
+  double zE = x.zS, cn = 0.0, qbn = x.qb;
+  x.next = !est;
+  if (stage == 4) {
+    StepState loc = st;
+    if (loc.active) end_step(loc, x.dz);
+    x.next = loc.active && !(loc.sched_n > 0 && loc.steps >= loc.sched_n);
+    zE = loc.zoff + loc.z;
+    if (rebased) qbn = loc.qbase;
+  } else if (stage != X_OPEN) {
+    zE = st.zoff + (st.z + (stage == 3 ? 1.0 : 0.5) * x.dz);
+    cn = stage == 3 ? x.dz : x.dz / 2;
+  }
+  x.zE = uniform_f64(zE);
+  x.qbn = uniform_f64(qbn);
+  x.cn = uniform_f64(cn);
+  return x;
+}
+
+// whether a stage-4 exchange forms max|q|: an adaptive run always, a fixed one on the step that ends the advance call
+// (see hankel_tile)
+__device__ __forceinline__ bool x_keeps_max(const StepState& st) {
+  return !(st.fixed && st.sub + 1 < st.sub_end && !(st.max_steps > 0 && st.steps + 1 >= st.max_steps));
+}
+
+// One point with a current (f < f1): its slope, S = 0.5 i exp(-i(kz+kg) z) J / Re kz (uppe.cl:73-91), the stage's
+// bookkeeping, and the next stage's input, which is returned. loc collects the largest step rate (stage 1 with est)
+// or the largest |q|^2 (stage 4).
+template <typename T>
+__device__ __forceinline__ cplx<T> x_slope(cplx<T> J, cplx<T> kz, double ph, cplx<T> Q, cplx<T> a1, cplx<T> a2,
+                                           cplx<T> a3, T cf, long idx, int stage, bool est, const XPos& x,
+                                           const StepState& st, double amin, cplx<T>* __restrict__ q,
+                                           cplx<T>* __restrict__ k1, cplx<T>* __restrict__ k2, cplx<T>* __restrict__ k3,
+                                           double& loc, bool& nan) {
+  const ColRef cr{x.zS - x.qb, x.qb, x.rb_end != 0};
+  const cplx<T> t = cmul(linear_factor<T>(ph, kz.im, x.zS, cr.za, -1), J);
+  cplx<T> S;
+  if constexpr (sizeof(T) == 4) {
+    const float rk = __builtin_amdgcn_rcpf(kz.re);  // 1 ulp
+    S = cmk(-0.5f * t.im * rk, 0.5f * t.re * rk);
+  } else {
+    S = cmk((T(-0.5) * t.im) / kz.re, (T(0.5) * t.re) / kz.re);
+  }
+  if (stage == 4) {
+    const T c6 = (T)(x.dz / 6), c3 = (T)(x.dz / 3);
+    T re = Q.re + c6 * a1.re;
+    T im = Q.im + c6 * a1.im;
+    re = re + c3 * a2.re;
+    im = im + c3 * a2.im;
+    re = re + c3 * a3.re;
+    im = im + c3 * a3.im;
+    re = re + c6 * S.re;
+    im = im + c6 * S.im;
+    cplx<T> v = cmk(re * cf, im * cf);
+    const double m2 = ref_update<T>(v, kz.im, cr, x.zS);
+    q[idx] = v;
+    loc = fmax(loc, m2);
+    return v;
+  }
+  cplx<T>* ks = stage == 1 ? k1 : (stage == 2 ? k2 : k3);
+  ks[idx] = S;
+  if (stage == 1) {
+    const double qr = (double)Q.re, qi = (double)Q.im;
+    if (qr != qr || qi != qi) nan = true;  // |q| is NaN exactly when a part is
+    if (est) {
+      // LoadStepSize (paraxial.cl:40-58), as in stage_point
+      const double sr = (double)S.re, si = (double)S.im;
+      const double am = ref_amin(amin, (double)kz.im, cr.qb);
+      const double rden = 1.0 / (qr * qr + qi * qi + am * am);
+      const double alpha = (qr * sr + qi * si) * rden;
+      const double keff = (qr * si - qi * sr) * rden;
+      loc = fmax(loc, 0.5 * st.dphi / st.L + fabs(keff) - alpha * (double)(alpha < 0.0));
+    }
+  }
+  const T ct = (T)x.cn;
+  return cscale(cmk(Q.re + ct * S.re, Q.im + ct * S.im), cf);
+}
+
+// the next stage's field from its input: linear propagation to its phase coordinate, and E = i kz A (UPPE)
+template <typename T>
+__device__ __forceinline__ cplx<T> x_field(cplx<T> v, cplx<T> kz, double ph, int f, const XPos& x, int env) {
+  v = cmul(linear_factor<T>(ph, kz.im, x.zE, f < x.f1r ? x.zE - x.qbn : x.zE, +1), v);
+  return env ? v : cmul(cmk(-kz.im, kz.re), v);
+}
+
 // one column tile: LAY its layout, RT its 16-row tiles per wave; LIN: a linear tile
 template <int CM, int RT, int LAY, bool LIN>
 __device__ __forceinline__ void x_tile(const XArgs<CM> a, int tile, int fc0, int hcw, char* smem, size_t slab_b) {
@@ -1533,34 +1635,14 @@ __device__ __forceinline__ void x_tile(const XArgs<CM> a, int tile, int fc0, int
 
   // ---- where this stage and the next one stand
   const StepState st = sw.take();
-  const double dz = uniform_f64(step_dz(st));
-  const double cs = stage == 4 ? 1.0 : (stage == X_OPEN || stage == 1 ? 0.0 : 0.5);
-  const double zS = uniform_f64(st.zoff + (st.z + cs * dz));
-  constexpr bool rebased = sizeof(T) == 4;  // only FP32 states are kept relative to a reference point
-  const double qb = uniform_f64(rebased ? st.qbase : 0.0);
-  const int rb_end = __builtin_amdgcn_readfirstlane(rebased && stage == 4 && rebase_at(st, st.zoff + (st.z + dz)));
-  const int f1r = rebased ? st.rb_f1 : 0;
-  double zE = zS, cn = 0.0, qbn = qb;
-  int next = !a.est;  // whether the next stage runs
-  if (stage == 4) {
-    StepState loc = st;
-    if (loc.active) end_step(loc, dz);
-    next = loc.active && !(loc.sched_n > 0 && loc.steps >= loc.sched_n);
-    zE = loc.zoff + loc.z;
-    if (rebased) qbn = loc.qbase;
-  } else if (stage != X_OPEN) {
-    zE = st.zoff + (st.z + (stage == 3 ? 1.0 : 0.5) * dz);
-    cn = stage == 3 ? dz : dz / 2;
-  }
-  zE = uniform_f64(zE);
-  qbn = uniform_f64(qbn);
-  const T ct = (T)uniform_f64(cn);
+  const XPos x = x_pos<T>(st, stage, a.est);
+  const int next = x.next;
   if (!st.active || (st.sched_n > 0 && st.steps >= st.sched_n)) {
     // the run has finished, or its schedule has (which the commit reports): nothing to update
     if (!LIN && st.active && stage == 4 && tid == 0 && tile == 0 && (blockIdx.z == 0 || a.zst)) a.st->pend = 1;
     return;
   }
-  const bool stays = (a.keep & (stage == 2 ? 1 : (stage == 4 ? 2 : 0))) && zE == zS;
+  const bool stays = (a.keep & (stage == 2 ? 1 : (stage == 4 ? 2 : 0))) && x.zE == x.zS;
   if (LIN && (stays || !next)) return;
 
   // ---- Hf . J
@@ -1581,7 +1663,6 @@ __device__ __forceinline__ void x_tile(const XArgs<CM> a, int tile, int fc0, int
   double loc = 0.0;  // stage 1: the largest step rate Kr; stage 4: the largest |q|^2
   bool nan = false;
   const double amin = a.est ? st.rel_amin * bitsd(*a.qmax) : 0.0;
-  const ColRef cr{zS - qb, qb, rb_end != 0};
 #pragma unroll
   for (int r = 0; r < RT; r++)
 #pragma unroll
@@ -1596,56 +1677,15 @@ __device__ __forceinline__ void x_tile(const XArgs<CM> a, int tile, int fc0, int
           const double php = ph[r][p];
           v = Qp;
           if (current && f < a.f1) {
-            // S = 0.5 i exp(-i(kz+kg) z) J / Re kz (uppe.cl:73-91)
-            const C t = cmul(linear_factor<T>(php, kzp.im, zS, cr.za, -1), J);
-            C S;
-            if constexpr (sizeof(T) == 4) {
-              const float rk = __builtin_amdgcn_rcpf(kzp.re);  // 1 ulp
-              S = cmk(-0.5f * t.im * rk, 0.5f * t.re * rk);
-            } else {
-              S = cmk((T(-0.5) * t.im) / kzp.re, (T(0.5) * t.re) / kzp.re);
-            }
-            if (stage == 4) {
-              const T c6 = (T)(dz / 6), c3 = (T)(dz / 3);
-              T re = Qp.re + c6 * a1[r][p].re;
-              T im = Qp.im + c6 * a1[r][p].im;
-              re = re + c3 * a2[r][p].re;
-              im = im + c3 * a2[r][p].im;
-              re = re + c3 * a3[r][p].re;
-              im = im + c3 * a3[r][p].im;
-              re = re + c6 * S.re;
-              im = im + c6 * S.im;
-              v = cmk(re * cf, im * cf);
-              const double m2 = ref_update<T>(v, kzp.im, cr, zS);
-              a.q[idx] = v;
-              loc = fmax(loc, m2);
-            } else {
-              C* ks = stage == 1 ? a.k1 : (stage == 2 ? a.k2 : a.k3);
-              ks[idx] = S;
-              if (stage == 1) {
-                const double qr = (double)Qp.re, qi = (double)Qp.im;
-                if (qr != qr || qi != qi) nan = true;  // |q| is NaN exactly when a part is
-                if (a.est) {
-                  // LoadStepSize (paraxial.cl:40-58), as in stage_point
-                  const double sr = (double)S.re, si = (double)S.im;
-                  const double am = ref_amin(amin, (double)kzp.im, cr.qb);
-                  const double rden = 1.0 / (qr * qr + qi * qi + am * am);
-                  const double alpha = (qr * sr + qi * si) * rden;
-                  const double keff = (qr * si - qi * sr) * rden;
-                  loc = fmax(loc, 0.5 * st.dphi / st.L + fabs(keff) - alpha * (double)(alpha < 0.0));
-                }
-              }
-              v = cscale(cmk(Qp.re + ct * S.re, Qp.im + ct * S.im), cf);
-            }
+            v = x_slope<T>(J, kzp, php, Qp, a1[r][p], a2[r][p], a3[r][p], cf, idx, stage, a.est, x, st, amin, a.q,
+                           a.k1, a.k2, a.k3, loc, nan);
           } else if (stage == X_OPEN2 && f < a.f1) {
+            const T ct = (T)x.cn;
             v = cscale(cmk(Qp.re + ct * a1[r][p].re, Qp.im + ct * a1[r][p].im), cf);
           } else if (stage != 4 && stage != X_OPEN) {
             v = cscale(Qp, cf);
           }
-          if (next) {
-            v = cmul(linear_factor<T>(php, kzp.im, zE, f < f1r ? zE - qbn : zE, +1), v);
-            if (!a.env) v = cmul(cmk(-kzp.im, kzp.re), v);  // E = i kz A
-          }
+          if (next) v = x_field<T>(v, kzp, php, f, x, a.env);
         }
         if (next && k < a.kpb && cl < hcw) x_put1<CM, LAY>(slab_e, a.kpb, k, cl, v);
       }
@@ -1654,8 +1694,7 @@ __device__ __forceinline__ void x_tile(const XArgs<CM> a, int tile, int fc0, int
       x_put1<CM, LAY>(slab_e, a.kpb, nwv * RT * 16 + e / hcw, e & (hcw - 1), cmk(T(0), T(0)));
 
   // max|q| for a later adaptive step (see hankel_tile), or the smallest step estimate
-  const bool red_on = current && (a.est || (stage == 4 && !(st.fixed && st.sub + 1 < st.sub_end &&
-                                                             !(st.max_steps > 0 && st.steps + 1 >= st.max_steps))));
+  const bool red_on = current && (a.est || (stage == 4 && x_keeps_max(st)));
   if (current && stage == 1 && nan) atomicOr(&a.st->nanflag, 1);
   if (red_on) {
     loc = a.est ? (loc > 0.0 ? st.dphi / loc : INFINITY) : sqrt(loc);
@@ -1914,6 +1953,121 @@ __global__ __launch_bounds__(1024) void f_tfft(
       if (blockIdx.x == 0 && blockIdx.y == 0) st->pend = 1;
     }
   }
+}
+
+// The last pass of one stage's forward transform and the first of the next stage's inverse one, both along y, in one
+// launch (the exchange of f_exchange on a Cartesian grid, stages 1 to 4): the forward pass leaves a line's slopes in
+// the workgroup that the inverse pass starts from, so q, kz and the phase table are read once where two launches read
+// them twice: per point and step 216 B in FP32 instead of 320 B. Bound by HBM at large grids. Adaptive runs take
+// stage 1 -> 2 as two launches of f_tfft.
+template <typename T, int CW>
+__global__ __launch_bounds__(1024) void f_texch(const cplx<T>* __restrict__ jr, cplx<T>* __restrict__ er, int na, int lg,
+                                                int nwp, int f1, int nw, const cplx<T>* __restrict__ tab_g, int tab_len,
+                                                T scale, const double* __restrict__ phs,
+                                                const cplx<T>* __restrict__ kzc, const T* __restrict__ cond,
+                                                cplx<T>* __restrict__ q, cplx<T>* __restrict__ k1,
+                                                cplx<T>* __restrict__ k2, cplx<T>* __restrict__ k3, StepState* stp,
+                                                unsigned long long* __restrict__ qmax_next, int stage, int env) {
+  using C = cplx<T>;
+  extern __shared__ __align__(16) char smem[];
+  C* buf = reinterpret_cast<C*>(smem);
+  C* tab = buf + na * CW;
+  __shared__ double red[16];
+  const int t = threadIdx.x, nth = blockDim.x, lane = t & 63, wave = t >> 6, nwv = nth >> 6;
+  const int f0 = blockIdx.x * CW;
+  const long base = (long)blockIdx.y * na * nwp + f0;
+  const int ne = na * CW;
+  const StateWords sw(stp);
+  __builtin_amdgcn_sched_barrier(0);
+  for (int i = t; i < tab_len; i += nth) tab[i] = tab_g[i];
+  const bool band = f0 < f1;  // a tile with a current
+  constexpr int LB = 4;       // elements per thread per batch, their loads issued together
+  if (band) {
+    for (int b0 = 0; b0 < ne; b0 += LB * nth) {
+      C v[LB];
+#pragma unroll
+      for (int j = 0; j < LB; j++) {
+        const int e = b0 + t + j * nth;
+        v[j] = cmk(T(0), T(0));
+        if (e < ne && f0 + e % CW < f1) v[j] = jr[base + (long)(e / CW) * nwp + e % CW];
+      }
+#pragma unroll
+      for (int j = 0; j < LB; j++) {
+        const int e = b0 + t + j * nth;
+        if (e < ne) buf[e] = v[j];
+      }
+    }
+  }
+  const StepState st = sw.take();
+  const XPos x = x_pos<T>(st, stage, false);
+  const bool first = blockIdx.x == 0 && blockIdx.y == 0;
+  if (!st.active || (st.sched_n > 0 && st.steps >= st.sched_n)) {
+    // the run has finished, or its schedule has (which the commit reports): nothing to update
+    if (st.active && stage == 4 && t == 0 && first) stp->pend = 1;
+    return;
+  }
+  __syncthreads();
+  if (band) lds_fft_cols<T, CW>(buf, na, lg, tab, -1);
+  double loc = 0.0;  // stage 4: the largest |q|^2
+  bool nan = false;
+  constexpr int EB = sizeof(T) == 8 ? 1 : 2;  // points per thread per batch
+  for (int b0 = 0; b0 < ne; b0 += EB * nth) {
+    C kz[EB], Q[EB], a1[EB], a2[EB], a3[EB];
+    double ph[EB];
+    T cf[EB];
+#pragma unroll
+    for (int j = 0; j < EB; j++) {
+      const int e = b0 + t + j * nth, f = f0 + e % CW;
+      if (e >= ne || f >= nw) continue;
+      const long idx = base + (long)(e / CW) * nwp + e % CW;
+      ph[j] = phs[idx];
+      kz[j] = kzc[idx];
+      Q[j] = q[idx];
+      cf[j] = cond[f];
+      if (stage == 4 && f < f1) {
+        a1[j] = k1[idx];
+        a2[j] = k2[idx];
+        a3[j] = k3[idx];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < EB; j++) {
+      const int e = b0 + t + j * nth, f = f0 + e % CW;
+      if (e >= ne) continue;
+      C v = cmk(T(0), T(0));
+      if (f < nw) {
+        const long idx = base + (long)(e / CW) * nwp + e % CW;
+        if (f < f1)
+          v = x_slope<T>(buf[e], kz[j], ph[j], Q[j], a1[j], a2[j], a3[j], cf[j], idx, stage, false, x, st, 0.0, q, k1,
+                         k2, k3, loc, nan);
+        else
+          v = stage == 4 ? Q[j] : cscale(Q[j], cf[j]);
+        if (x.next) v = x_field<T>(v, kz[j], ph[j], f, x, env);
+      }
+      buf[e] = v;
+    }
+  }
+  const bool red_on = stage == 4 && x_keeps_max(st);
+  if (stage == 1 && nan) atomicOr(&stp->nanflag, 1);
+  if (red_on) {
+    loc = sqrt(loc);
+    for (int o = 32; o > 0; o >>= 1) loc = fmax(loc, __shfl_xor(loc, o));
+    if (lane == 0) red[wave] = loc;
+  }
+  __syncthreads();
+  if (t == 0) {
+    if (red_on) {
+      double v = red[0];
+      for (int i = 1; i < nwv; i++) v = fmax(v, red[i]);
+      atomicMax(&qmax_next[red_slot(blockIdx.x + gridDim.x * blockIdx.y)], dbits(v));
+    }
+    // the step has run; the next step's stage-1 source launch commits its end
+    if (stage == 4 && first) stp->pend = 1;
+  }
+  if (!x.next) return;
+  lds_fft_cols<T, CW>(buf, na, lg, tab, +1);
+  for (int e = t; e < ne; e += nth)
+    if (f0 + e % CW < nw) er[base + (long)(e / CW) * nwp + e % CW] = cscale(buf[e], scale);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -4303,26 +4457,55 @@ struct Fused {
             zfix, s->qbase, s->f1);
   }
 
-  // one RK4 step on a Cartesian grid: per RHS, the inverse transform (y with the stage prologue, then x), the
-  // source, the forward transform over the nonlinear band (x, then y with the RK stage epilogue)
-  static void step_cart(uppe_handle* h, FusedState* s) {
+  // the exchange of `stage` along y: J_r after its x pass to the next stage's field before its own
+  template <int CW>
+  static void texch(uppe_handle* h, FusedState* s, int stage) {
+    const int na = h->n2, nth = std::max(64, CW * std::max(1, na / 8));
+    const dim3 grid((unsigned)((h->nw + CW - 1) / CW), (unsigned)h->n1);
+    const size_t shm = sizeof(C) * ((size_t)na * CW + s->twlen_y);
+    if (nth > 1024 || shm > kMaxLds) throw Error{UPPE_ERR_UNSUPPORTED, "transverse pass: line too long"};
+    launchf(h, UPPE_KC_EXCHANGE, f_texch<T, CW>, grid, dim3(nth), shm, (const C*)s->jr, (C*)s->er, na, ilog2i(na),
+            s->nwp, s->f1, h->nw, (const C*)s->tw_y, s->twlen_y, T(1.0 / na), (const double*)s->phs, (const C*)s->kzc,
+            (const T*)s->cond, (C*)s->q, (C*)s->k1, (C*)s->k2, (C*)s->k3, s->st, s->qmax_next, stage,
+            h->paraxial ? 1 : 0);
+  }
+
+  // One RK4 step on a Cartesian grid: per RHS, the x pass of the inverse transform, the source, the x pass of the
+  // forward transform over the nonlinear band, and the y passes of the forward and of the next stage's inverse
+  // transform in one launch. `first` and `known` as for step_mfma: a run opens with a y pass of its own, and an
+  // adaptive one takes stage 1's y passes one by one.
+  static void step_cart(uppe_handle* h, FusedState* s, bool first, bool known) {
     const C* kp[5] = {nullptr, nullptr, (const C*)s->k1, (const C*)s->k2, (const C*)s->k3};
     C *q = (C*)s->q, *er = (C*)s->er, *jr = (C*)s->jr;
-    for (int stage = 1; stage <= 4; stage++) {
+    auto open = [&](int stage) {
       if (h->paraxial)
         tpass<PRO_STAGE_ENV, EPI_NONE>(h, s, 2, q, er, h->nw, +1, kp[stage], stage, 0.0, s->st);
       else
         tpass<PRO_STAGE, EPI_NONE>(h, s, 2, q, er, h->nw, +1, kp[stage], stage, 0.0, s->st);
+    };
+    if (first) open(1);
+    for (int stage = 1; stage <= 4; stage++) {
       tpass<PRO_NONE, EPI_NONE>(h, s, 1, er, er, h->nw, +1, nullptr, stage, 0.0, s->st);
       source(h, s, er, jr, false, stage == 1 ? s->st : nullptr);
       tpass<PRO_NONE, EPI_NONE>(h, s, 1, jr, jr, s->f1, -1, nullptr, stage, 0.0, s->st);
-      tpass<PRO_NONE, EPI_STAGE>(h, s, 2, jr, (C*)nullptr, s->f1, -1, nullptr, stage, 0.0, s->st);
+      if (stage == 1 && !known) {
+        tpass<PRO_NONE, EPI_STAGE>(h, s, 2, jr, (C*)nullptr, s->f1, -1, nullptr, stage, 0.0, s->st);
+        open(2);
+        continue;
+      }
+      if constexpr (sizeof(T) == 4) {
+        if (h->n2 <= 512) {
+          texch<16>(h, s, stage);
+          continue;
+        }
+      }
+      texch<8>(h, s, stage);
     }
   }
 
   static void step(uppe_handle* h, FusedState* s, bool first, bool known) {
     if (h->d.geometry == UPPE_CARTESIAN) {
-      step_cart(h, s);
+      step_cart(h, s, first, known);
       return;
     }
     if (s->cm >= 0) {

@@ -1,7 +1,9 @@
-'''The exchange launches of radial grids (r2k contraction of one stage and k2r contraction of the next in one kernel)
-at the edges of their tiles, against the oracle: fewer rows than a 16-row tile, modes that end inside one, nonlinear
-bands that end inside a column tile, both tile widths, one to four row tiles per wave. Every grid runs fixed, adaptive
-and replayed steps in two advance calls, so each stage opens, exchanges and resumes. Tolerances as for the other parity
+'''The exchange launches (the transform of one stage back to k-space and the next stage's transform out of it in one
+kernel) at the edges of their tiles, against the oracle. Radial grids: fewer rows than a 16-row tile, modes that end
+inside one, nonlinear bands that end inside a column tile, both tile widths, one to four row tiles per wave. Cartesian
+grids: the shortest lines, lines of every first radix, the longest (8 FP32 columns per line), bands that end inside a
+column tile. Every grid runs fixed, adaptive and replayed steps in two advance calls, so each stage opens, exchanges and
+resumes. Tolerances as for the other parity
 tests: FP64 1e-10, FP32 and BF16x3 1e-5 on the oracle's steps.
 '''
 import sys
@@ -19,6 +21,9 @@ GRIDS = [(129, 8, 5, 1.0), (129, 16, 16, 0.61), (257, 32, 27, 0.43), (257, 128, 
 # two 16-row tiles per wave on half tiles (BF16x3), four (FP64)
 TALL = [(257, 512, 491, 1.0, 'bf16x3'), (1025, 512, 300, 1.0, 'fp64')]
 
+# Cartesian: (frequencies, x cells, y cells, share of the band that is nonlinear)
+LINES = [(33, 4, 2, 1.0), (33, 2, 8, 0.5), (65, 8, 16, 0.4), (33, 4, 128, 1.0), (17, 2, 1024, 0.7)]
+
 _refs = {}
 
 
@@ -29,6 +34,17 @@ def _vol(nw, nr, nk, share):
     band = (0.0, max(2.0, vol['frequency band'][1]))
     vol['frequency band'] = band
     vol['nonlinear band'] = (0.0, max(1.4, share * band[1]))
+    return vol
+
+
+def _lines_vol(nw, nx, ny, share):
+    vol = configs.cartesian_filamentation(scale=8, steps=100, length='10 cm')
+    vol['wave grid'] = (nw, nx, ny, 2)
+    vol['frequency band'] = (0.0, 2.0)
+    vol['nonlinear band'] = (0.0, 2.0 * share)
+    vol['minimum step'] = 1.0
+    vol['size'] = vol['size'][:2] + (vol['size'][2] * 3 / 100,)
+    vol['subcycles'] = 3
     return vol
 
 
@@ -45,9 +61,9 @@ def _run(rs, factory, mode, schedule=None):
         return st.get_state(), recs
 
 
-def _check(oracle_mod, grid, precision):
+def _check(oracle_mod, grid, precision, build=_vol):
     if grid not in _refs:
-        rs = uppe_kernel.RunSetup(_vol(*grid))
+        rs = uppe_kernel.RunSetup(build(*grid))
         _refs[grid] = rs, {m: _run(rs, oracle_mod.oracle_factory, m) for m in ('fixed', 'adaptive')}
     rs, refs = _refs[grid]
     factory = uppe_kernel.hip_stepper_factory(precision)
@@ -69,3 +85,9 @@ def test_exchange_tiles(oracle_mod, grid, precision):
 @pytest.mark.parametrize('case', TALL)
 def test_exchange_row_tiles(oracle_mod, case):
     _check(oracle_mod, case[:4], case[4])
+
+
+@pytest.mark.parametrize('grid', LINES)
+@pytest.mark.parametrize('precision', ['fp64', 'fp32'])
+def test_exchange_lines(oracle_mod, grid, precision):
+    _check(oracle_mod, grid, precision, _lines_vol)
