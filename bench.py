@@ -354,9 +354,8 @@ def batch_workload(prec, K, W, seq_steps, graph_steps=8):
 def cartesian_workload(prec, K, W, compare=True, cpu=False):
     '''The 3-D Cartesian filamentation workload (Nw = 513, 256 x 256 over 4 mm x 4 mm, 20 P_cr super-Gaussian
     beam with 10 % amplitude noise, Kerr + O2 photoionisation, 200 fixed steps over 10 cm): K timed steps on one
-    handle, per-kernel-class averages with HIP events and the roofline of the transverse FFT pass (28 B per grid
-    point per launch in FP32: 40 B on the passes with the stage prologue or epilogue, 16 B on the plain ones), the
-    plain FP64 stepper and the fused FP64 stepper (whose state after 3 steps gives the error), and with cpu the FP64
+    handle, per-kernel-class averages with HIP events and the roofline of the exchange (the y passes around the RK
+    stage in one launch: 54 B per grid point on the average of the four stages in FP32), the plain FP64 stepper and the fused FP64 stepper (whose state after 3 steps gives the error), and with cpu the FP64
     oracle on one step of the host cores.'''
     vol = configs.cartesian_filamentation()
     rs = uppe_kernel.RunSetup(vol)
@@ -368,17 +367,20 @@ def cartesian_workload(prec, K, W, compare=True, cpu=False):
     n, secs, _ = run_steps(rs, st, K)
     st.profile_enable(True)
     run_steps(rs, st, min(K, 10))
-    classes = {kc: st.profile_read(kc) for kc in ('transverse_fft', 'source', 'reduce')}
+    classes = {kc: st.profile_read(kc) for kc in ('exchange', 'transverse_fft', 'source', 'reduce')}
     st.profile_enable(False)
     st.close()
     el = 8 if prec.startswith('fp64') else 4
-    ms, cnt = classes['transverse_fft']
+    # a stepper without exchanges (plain FP64): the transverse passes, 28 B on their average
+    kc, kname, per_pt = (('exchange', 'f_texch (y passes of a stage and the next, with the RK stage)', 54.0)
+                         if classes['exchange'][1] else ('transverse_fft', 'transverse FFT pass', 28.0))
+    ms, cnt = classes[kc]
     avg_s = ms / max(cnt, 1) * 1e-3
-    B = 28.0 * (el / 4) * pts
+    B = per_pt * (el / 4) * pts
     out = dict(value=pts * n / secs, steps=n, ms_per_step=1e3 * secs / n, precision=prec,
                workload='3-D Cartesian filamentation, Nw=513, 256x256 over 4 mm, Kerr + O2, 200 fixed steps over '
                         '10 cm; first %d steps' % n,
-               roofline=dict(bound='hbm', kernel='f_tfft (transverse FFT pass)', achieved=B / avg_s / 1e9,
+               roofline=dict(bound='hbm', kernel=kname, achieved=B / avg_s / 1e9,
                              peak=HBM_PEAK_GBS, unit='GB/s', frac=B / avg_s / 1e9 / HBM_PEAK_GBS, traffic=None,
                              avg_launch_us=avg_s * 1e6, launches=cnt, bytes_per_launch=B),
                class_avg_us={k: (v[0] / v[1] * 1e3 if v[1] else None) for k, v in classes.items()})
