@@ -59,6 +59,23 @@ class AnalyticBox:
         for suffix, arr in zip(names, arrays):
             np.save(basename + '_' + self.name + '_' + suffix, arr)
 
+    def GetRelDensityPlanes(self, xp, zs):
+        '''GetRelDensity of the points xp (N1, N2, 8) moved to each z of zs, in one evaluation of the density lambda:
+        an array (len(zs), N1, N2), or None where the lambda does not map positions to densities of their shape (one
+        that returns a plain number, or changes its arguments in place).'''
+        zs = np.asarray(zs, dtype=float)
+        shape = zs.shape + xp.shape[:2]
+
+        def planes(a):
+            return np.broadcast_to(a, shape)
+        r2 = np.einsum('...i,...i', xp[..., 1:3], xp[..., 1:3])
+        try:
+            dens = np.asarray(self.vol_dict['density lambda'](planes(xp[..., 1]), planes(xp[..., 2]),
+                                                              planes(zs[:, None, None]), planes(r2)), dtype=float)
+        except (ValueError, TypeError, IndexError):
+            return None
+        return dens if dens.shape == shape else None
+
     def GetRelDensity(self, xp):
         x = xp[..., 1]
         y = xp[..., 2]
