@@ -2195,7 +2195,19 @@ template <>
 __device__ inline double ion_rate<double>(double ea, const uppe_ionization& ion, double log_pre) {
   if (ion.kind == UPPE_ION_EXPLICIT) {
     double emag = ion.e_conv * ea + ion.e_cutoff;
-    return ion.rate_conv * ion.c_pre * pow(emag, ion.c_pow) * exp(ion.c_exp / emag);
+    const double pre = ion.rate_conv * ion.c_pre;
+    // (also false for NaN; the product below would turn 0 and infinity into NaN)
+    if (!(emag > 1e-280 && emag < 1e280)) return pre * pow(emag, ion.c_pow) * exp(ion.c_exp / emag);
+    // The two factors as one exponential of c_pow log E + c_exp / E, the quotient by a Newton step on the hardware
+    // reciprocal. What the quotient, the product and the sum round off is carried and applied to first order, so that
+    // the exponent's error is the logarithm's alone; a rounded c_exp / E alone costs half an ulp times its size.
+    double y = __builtin_amdgcn_rcp(emag);
+    y = fma(y, fma(-emag, y, 1.0), y);
+    const double q = ion.c_exp * y, ql = fma(-q, emag, ion.c_exp) * y;
+    const double lg = log(emag), p = ion.c_pow * lg, pl = fma(ion.c_pow, lg, -p);
+    const double x = q + p, b = x - q, xl = (q - (x - b)) + (p - b) + (ql + pl);
+    const double r = exp(x);
+    return pre * (r > 0.0 && r < INFINITY ? fma(r, xl, r) : r);
   }
   double lg = log(ion.e_conv * ea + ion.e_cutoff);
   return ion.rate_conv * exp(ion.c[0] + ion.c[1] * lg + ion.c[2] * lg * lg + ion.c[3] * (lg * lg * lg) +
@@ -2586,7 +2598,9 @@ __global__ __launch_bounds__(1024) void f_source(const cplx<T>* __restrict__ er,
   // then this strip's spectrum and the frequency and filter of the bins this thread writes at the end. The tables
   // come from L2 and reach LDS while the strip is still on its way from HBM.
   // Per-pass twiddle tables of the N- and N/2-point transforms (fewer than N + N/2 entries): in LDS for FP32
-  // strips up to 4096 samples, read from L2 for FP64 and the 8192-sample strips (LDS would not fit)
+  // strips up to 4096 samples, read from L2 for the 8192-sample strips (LDS would not fit) and for FP64, where
+  // staging them takes longer than the passes gain (128 strips of 1024 samples: 1.5 us against 0.6; 2048 of
+  // 256: 4.4 against 0.7)
   constexpr bool kTabLds = sizeof(T) == 4 && SPT <= 4;
   constexpr int TPT = kTabLds ? (3 * SPT + 1) / 2 : 1;  // table entries per thread: tlen < N + N/2 = 1.5 SPT nth
   const int tlen = r8_table_len(lgn) + r8_table_len(lgm);
@@ -3752,14 +3766,15 @@ static bool wave_source_forced() {
   return env && env[0] == '2';
 }
 
-// the FP32 stepping source kernel (no diagnostics, no rotator) for Nt = 2^LG, where the block of Nt / S threads
-// fits 64..1024; otherwise the kernel for any Nt
-template <int S, int LG>
+// the stepping source kernel (no diagnostics, no rotator) for Nt = 2^LG, where the block of Nt / S threads fits
+// 64..1024; otherwise the kernel for any Nt. FP64 at 128 strips, launch 15.4 -> 11 us (2048 samples, O2), 8.0 -> 6.4
+// (1024, Kerr), the rate as one exponential and the twiddles requested early among them.
+template <typename T, int S, int LG>
 constexpr auto source_fixed() {
   if constexpr ((1 << LG) / S <= 1024 && (1 << LG) / S >= 64)
-    return f_source<float, S, false, false, LG>;
+    return f_source<T, S, false, false, LG>;
   else
-    return f_source<float, S, false, false, 0>;
+    return f_source<T, S, false, false, 0>;
 }
 
 // the same for the FP32 envelope source kernel (Nt = Nw = 256 .. 1024)
@@ -4188,7 +4203,17 @@ struct Fused {
                     : (diag ? f_source<T, S, true, false> : f_source<T, S, false, false>);                      \
     if constexpr (sizeof(T) == 4 && S <= 4)                                                                      \
       if (!rot && !diag && lgn >= 10 && lgn <= 12)                                                               \
-        kern = lgn == 10 ? source_fixed<S, 10>() : (lgn == 11 ? source_fixed<S, 11>() : source_fixed<S, 12>());  \
+        kern = lgn == 10   ? source_fixed<T, S, 10>()                                                            \
+               : lgn == 11 ? source_fixed<T, S, 11>()                                                            \
+                           : source_fixed<T, S, 12>();                                                           \
+    if constexpr (sizeof(T) == 8 && S <= 4)                                                                      \
+      if (!rot && !diag && lgn >= 7 && lgn <= 12)                                                                \
+        kern = lgn == 7    ? source_fixed<T, S, 7>()                                                             \
+               : lgn == 8  ? source_fixed<T, S, 8>()                                                             \
+               : lgn == 9  ? source_fixed<T, S, 9>()                                                             \
+               : lgn == 10 ? source_fixed<T, S, 10>()                                                            \
+               : lgn == 11 ? source_fixed<T, S, 11>()                                                            \
+                           : source_fixed<T, S, 12>();                                                           \
     launchf(h, UPPE_KC_SOURCE, kern, grid_src, block, shm, er, jr, diag ? (T*)s->chi_t : (T*)nullptr,             \
             diag ? (T*)s->ne_t : (T*)nullptr, (const C*)s->tw, (const T*)s->w, (const T*)s->nlf,                  \
             (const double*)s->ng, N, lgn, s->nwp, s->redchi3, s->dt, s->ion, log_pre,                             \

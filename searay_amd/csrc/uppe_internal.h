@@ -223,18 +223,24 @@ __device__ __forceinline__ void lds_fft_r8(cplx<T>* buf, int n_rt, int lg_rt, co
     Ns = R;
   }
   const cplx<T>* tp = tab;
+  // FP64 tables are read from L2: a pass requests its twiddles with its points, ahead of the barrier
+  constexpr bool PRE = sizeof(T) == 8;
   auto pass = [&](int Ns) {
     const int nb = n >> 3;
-    cplx<T> v[8], y[8];
-    if (tid < nb)
+    cplx<T> v[8], y[8], tw[PRE ? 8 : 1];
+    const int k = tid & (Ns - 1);
+    if (tid < nb) {
+      if constexpr (PRE)
+#pragma unroll
+        for (int r = 1; r < 8; r++) tw[r] = tp[(r - 1) * Ns + k];
 #pragma unroll
       for (int r = 0; r < 8; r++) v[r] = buf[lds_swz<T>(tid + r * nb)];
+    }
     __syncthreads();
     if (tid < nb) {
-      const int k = tid & (Ns - 1);
 #pragma unroll
       for (int r = 1; r < 8; r++) {
-        cplx<T> w = tp[(r - 1) * Ns + k];
+        cplx<T> w = PRE ? tw[PRE ? r : 0] : tp[(r - 1) * Ns + k];
         if (sign > 0) w.im = -w.im;
         v[r] = cmul(v[r], w);
       }
