@@ -19,6 +19,7 @@
 #include "uppe_internal.h"
 
 #include <algorithm>
+#include <complex>
 #include <cstring>
 #include <mutex>
 #include <type_traits>
@@ -188,6 +189,18 @@ struct RotRow {
   T c, wr, wi, pad;
   cplx<T> e[2 + ROT_NB];
 };
+
+// The constants of one state for the SPT samples of a thread in rot_chi, which follow the rows of all
+// states (padded with zeros to whole groups of rot_group): with
+// W_j dt = w and m = SPT t + i, e_i = E^(2i+1), b_i = c w conj(E^(2i)) and k_il = c Re(E^(2l+1) conj(E^(2i)) w), l < i
+// (row i from i (i - 1) / 2). After those of all states, ROT_POW powers a state: E^(2 SPT l) of lane l, then
+// E^(2 SPT 64 v) of wave v, whose product starts thread 64 v + l.
+template <typename T, int SPT>
+struct RotFwd {
+  cplx<T> e[SPT], b[SPT];
+  T k[SPT > 1 ? SPT * (SPT - 1) / 2 : 1];
+};
+constexpr int ROT_POW = 64 + 16;
 
 constexpr int BM = 64, BN = 64, BK = 16;
 
@@ -2367,10 +2380,63 @@ __device__ inline cplx<double> rot_start<double>(const RotRow<double>& rw, int t
   return pw;
 }
 
-// rotator states whose constants are staged in LDS at a time
-constexpr int ROT_CHUNK = 64;
-// rotator states per barrier in the source kernel
-constexpr int ROT_G32 = 8, ROT_G64 = 2;
+// rotator states per barrier in the source kernel and in its adjoint
+constexpr int ROT_G32 = 8, ROT_G64 = 4, ROT_ADJ_G64 = 2;
+template <typename T>
+constexpr int rot_group() {
+  return sizeof(T) == 4 ? ROT_G32 : ROT_G64;
+}
+
+// rotator states whose constants are staged in LDS at a time: whole groups, at most 64, in 8 KB (a strip of 8192 FP64
+// samples leaves 32 KB of LDS)
+template <typename T, int SPT>
+constexpr int rot_chunk() {
+  constexpr int fit = 8192 / (int)sizeof(RotFwd<T, SPT>);
+  return (fit < 64 ? fit : 64) / rot_group<T>() * rot_group<T>();
+}
+
+// wave_excl_prefix of N values, and lanes_below, step by step side by side
+template <typename T, int N>
+__device__ __forceinline__ void wave_excl_prefix_all(T (&v)[N]) {
+  auto step = [&](auto ctrl, auto rows, bool add) {
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      const T m = dpp_move<decltype(ctrl)::value, decltype(rows)::value>(v[i]);
+      v[i] = add ? v[i] + m : m;
+    }
+  };
+  std::integral_constant<int, 0xf> all;
+  step(std::integral_constant<int, 0x138>(), all, false);
+  step(std::integral_constant<int, 0x111>(), all, true);
+  step(std::integral_constant<int, 0x112>(), all, true);
+  step(std::integral_constant<int, 0x114>(), all, true);
+  step(std::integral_constant<int, 0x118>(), all, true);
+  step(std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xa>(), true);
+  step(std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xc>(), true);
+}
+template <typename T, int N>
+__device__ __forceinline__ void lanes_below_all(T (&v)[N], int k) {
+  auto step = [&](auto ctrl) {
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] += dpp_move<decltype(ctrl)::value, 0xf>(v[i]);
+  };
+  step(std::integral_constant<int, 0x111>());
+  step(std::integral_constant<int, 0x112>());
+  step(std::integral_constant<int, 0x114>());
+  step(std::integral_constant<int, 0x118>());
+  const int last = (k - 1) & 15;
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    if constexpr (sizeof(T) == 4) {
+      const int b = __builtin_amdgcn_readlane(__float_as_int(v[i]), last);
+      v[i] = __int_as_float(k == 0 ? 0 : b);
+    } else {
+      const long long w = __double_as_longlong(v[i]);
+      const int lo = __builtin_amdgcn_readlane((int)w, last), hi = __builtin_amdgcn_readlane((int)(w >> 32), last);
+      v[i] = __longlong_as_double(k == 0 ? 0ll : ((long long)hi << 32) | (unsigned int)lo);
+    }
+  }
+}
 
 // Rotational (Raman) susceptibility on the SPT samples a thread owns (rotations.cl:26-129, AddChiUPPE and
 // AddChiParaxial). For each state j >= 2 the reference runs the recurrence rho <- rho - i dt F_m E^(2m+1) and
@@ -2379,85 +2445,135 @@ constexpr int ROT_G32 = 8, ROT_G64 = 2;
 // |E|^2 / 2 for the envelope. Both running sums are prefix sums over m, and the thread order already follows m:
 // rho_m is a DPP wave scan plus the totals of the earlier waves, one barrier per G states. The sum over states
 // commutes with the outer prefix sum, so the per-state terms g_j(m) are summed first and scanned once.
+//
+// The kernel is bound by its instructions on one wave per SIMD, so a state costs few per sample. With P the start
+// power E^(2m) of the thread's first sample and B the sum over the threads before it, the sum ahead of sample i is
+// r_i = B + P sum_{l < i} F_l E^(2l+1), and the state's term is the real part of
+//   (B conj(P)) (w conj(E^(2i))) + |P|^2 sum_{l < i} F_l E^(2l+1) conj(E^(2i)) w
+// times -c n_g dt: one complex product per thread and two multiply-adds per sample, plus the second sum, whose
+// factors are constants (RotFwd). Running both recurrences sample by sample instead took about twice the
+// instructions, a third of them for the start powers (FP64 phases and the hardware sine, cosine and exponential; ten
+// products in FP64), which are now the product of two table entries. 30 states on 256 FP32 strips of 1024 samples:
+// 16.0 -> 10.0 us of the launch.
+//
+// Nothing in the loop over groups branches (the rows are padded to whole groups with zeros), so that the scans of a
+// group's states interleave: with one wave per SIMD a chain of dependent lane moves otherwise waits for each of them
+// (15.2 us). The tables are read through the constant address space: a batch's pointers would make flat loads
+// of them, which the group's LDS reads would wait for.
 template <typename R, int SPT>
 __device__ inline void rot_chi(const R* drive, R ngp, R* dchi, const RotRow<R>* __restrict__ rot_tab, int rot_states,
-                               double rot_fc, double dt, int N, int a0) {
-  const int tid = threadIdx.x, nth = blockDim.x, lane = tid & 63, wave = tid >> 6, nwv = nth >> 6;
+                               double rot_fc, double dt) {
+  using Fwd = RotFwd<R, SPT>;
+  typedef R vec2 __attribute__((ext_vector_type(2)));
+  typedef const __attribute__((address_space(4))) vec2* pow_ptr;
+  typedef const __attribute__((address_space(4))) unsigned* word_ptr;
+  constexpr int G = rot_group<R>();  // states per barrier
+  constexpr int CHUNK = rot_chunk<R, SPT>();
+  static_assert(CHUNK >= G, "a group's constants fit the staging buffer");
+  const int tid = threadIdx.x, nth = blockDim.x, lane = tid & 63, wave = tid >> 6;
   __shared__ R rot_wsr[16];
-  constexpr int G = sizeof(R) == 4 ? ROT_G32 : ROT_G64;  // states per barrier
-  const R dtr = (R)dt, fc = (R)rot_fc;
-  const int m0 = N - a0 - SPT;  // = SPT tid: m of this thread's last sample; m grows as the sample index falls
+  const int n = rot_states - 2, np = (n + G - 1) / G * G;
+  const Fwd* fwd = reinterpret_cast<const Fwd*>(rot_tab + n);
+  const pow_ptr pows = (pow_ptr)(const vec2*)(fwd + np);
   const int wv_u = __builtin_amdgcn_readfirstlane(wave);
-  R gs[SPT];
+  // sample i of the thread in order of m: index SPT - 1 - i of drive and dchi
+  R F[SPT], gs[SPT];
 #pragma unroll
-  for (int j = 0; j < SPT; j++) gs[j] = R(0);
-  // per-state constants, staged in LDS for ROT_CHUNK states at a time; the wave totals of G states per
+  for (int i = 0; i < SPT; i++) {
+    F[i] = (R)rot_fc * drive[SPT - 1 - i];
+    gs[i] = R(0);
+  }
+  vec2 pl[G], pv[G];
+  auto load_pows = [&](int q0) {
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      const pow_ptr pq = pows + (long)(q0 + g) * ROT_POW;
+      pl[g] = pq[lane];
+      pv[g] = pq[64 + wv_u];
+    }
+  };
+  load_pows(0);
+  // per-state constants, staged in LDS for CHUNK states at a time; the wave totals of G states per
   // barrier, double-buffered
-  __shared__ RotRow<R> rot_r[ROT_CHUNK];
+  __shared__ Fwd rot_r[CHUNK];
   __shared__ cplx<R> rot_ws[2][G][16];
   int par = 0;
-  for (int s0 = 2; s0 < rot_states; s0 += ROT_CHUNK) {
-    const int nc = min(ROT_CHUNK, rot_states - s0);
+  for (int s0 = 0; s0 < np; s0 += CHUNK) {
+    const int nc = min(CHUNK, np - s0);
     __syncthreads();  // the previous chunk's constants are no longer read
     {
-      const unsigned* src = reinterpret_cast<const unsigned*>(rot_tab + (s0 - 2));
+      const word_ptr src = (word_ptr)reinterpret_cast<const unsigned*>(fwd + s0);
       unsigned* dst = reinterpret_cast<unsigned*>(rot_r);
-      const int words = nc * (int)(sizeof(RotRow<R>) / sizeof(unsigned));
+      const int words = nc * (int)(sizeof(Fwd) / sizeof(unsigned));
       for (int i = tid; i < words; i += nth) dst[i] = src[i];
     }
     __syncthreads();
     for (int q0 = 0; q0 < nc; q0 += G) {
+      // the start powers of this group, and the next group's on their way (the last group's again, not used)
+      cplx<R> P[G], tot[G];
+#pragma unroll
+      for (int g = 0; g < G; g++) P[g] = cmul(cmk(pl[g].x, pl[g].y), cmk(pv[g].x, pv[g].y));
+      load_pows(min(s0 + q0 + G, np - G));
       // pass 1: this thread's sum of F_m E^(2m+1), its exclusive scan over the wave, the wave totals
-      cplx<R> pw0[G], run[G];
+      R run[2 * G];
 #pragma unroll
       for (int g = 0; g < G; g++) {
-        const RotRow<R>& rw = rot_r[min(q0 + g, nc - 1)];  // past the chunk end: a repeat, not used
-        const cplx<R> e1 = rw.e[0], e2 = rw.e[1];
-        cplx<R> pw = rot_start(rw, tid, m0), tot = cmk(R(0), R(0));
-        pw0[g] = pw;
+        const Fwd& rw = rot_r[q0 + g];
+        cplx<R> t = cscale(rw.e[0], F[0]);
 #pragma unroll
-        for (int jj = SPT - 1; jj >= 0; jj--) {
-          tot = cadd(tot, cscale(cmul(pw, e1), fc * drive[jj]));
-          pw = cmul(pw, e2);
-        }
-        run[g] = cmk(wave_excl_prefix(tot.re), wave_excl_prefix(tot.im));
-        if (lane == 63) rot_ws[par][g][wave] = cadd(run[g], tot);
+        for (int i = 1; i < SPT; i++) t = cadd(t, cscale(rw.e[i], F[i]));
+        tot[g] = cmul(P[g], t);
+        run[2 * g] = tot[g].re;
+        run[2 * g + 1] = tot[g].im;
       }
+      wave_excl_prefix_all(run);
+      if (lane == 63)
+#pragma unroll
+        for (int g = 0; g < G; g++) rot_ws[par][g][wave] = cadd(cmk(run[2 * g], run[2 * g + 1]), tot[g]);
       __syncthreads();
-      // pass 2: rho_m = -i dt (sum of F E^(2m+1) over earlier m); g_j(m) = c_j Im(rho conj(E^(2m)) W dt)
+      // pass 2: the sums of the earlier waves (lanes from the wave's own on are not used), then the states' terms
+      R low[2 * G];
 #pragma unroll
       for (int g = 0; g < G; g++) {
-        if (q0 + g < nc) {
-          const RotRow<R>& rw = rot_r[q0 + g];
-          const R cj = rw.c * ngp, wr = rw.wr, wi = rw.wi;
-          const cplx<R> e1 = rw.e[0], e2 = rw.e[1];
-          const cplx<R> wt = lane < nwv ? rot_ws[par][g][lane] : cmk(R(0), R(0));
-          cplx<R> r = cadd(run[g], cmk(lanes_below(wt.re, wv_u), lanes_below(wt.im, wv_u)));
-          cplx<R> pw = pw0[g];
+        const cplx<R> wt = rot_ws[par][g][lane & 15];
+        low[2 * g] = wt.re;
+        low[2 * g + 1] = wt.im;
+      }
+      lanes_below_all(low, wv_u);
 #pragma unroll
-          for (int jj = SPT - 1; jj >= 0; jj--) {
-            const cplx<R> rho = cmk(dtr * r.im, -dtr * r.re);
-            const cplx<R> qv = cmul(rho, cconj(pw));
-            gs[jj] += cj * (qv.re * wi + qv.im * wr);
-            r = cadd(r, cscale(cmul(pw, e1), fc * drive[jj]));
-            pw = cmul(pw, e2);
+      for (int g = 0; g < G; g++) {
+        const Fwd& rw = rot_r[q0 + g];
+        const cplx<R> z = cmul(cmk(run[2 * g] + low[2 * g], run[2 * g + 1] + low[2 * g + 1]), cconj(P[g]));
+        const R p2 = P[g].re * P[g].re + P[g].im * P[g].im;
+#pragma unroll
+        for (int i = 0; i < SPT; i++) {
+          gs[i] += z.re * rw.b[i].re - z.im * rw.b[i].im;
+          if (i > 0) {
+            R own = F[0] * rw.k[i * (i - 1) / 2];
+#pragma unroll
+            for (int l = 1; l < i; l++) own += F[l] * rw.k[i * (i - 1) / 2 + l];
+            gs[i] += p2 * own;
           }
         }
       }
       par ^= 1;
     }
   }
+  const R sc = -(R)dt * ngp;
   R gtot = R(0);
 #pragma unroll
-  for (int jj = 0; jj < SPT; jj++) gtot += gs[jj];
+  for (int i = 0; i < SPT; i++) {
+    gs[i] *= sc;
+    gtot += gs[i];
+  }
   R cum = wave_excl_prefix(gtot);
   if (lane == 63) rot_wsr[wave] = cum + gtot;
   __syncthreads();
-  cum += lanes_below(lane < nwv ? rot_wsr[lane] : R(0), wv_u);  // the earlier waves' totals
+  cum += lanes_below(lane < (nth >> 6) ? rot_wsr[lane] : R(0), wv_u);  // the earlier waves' totals
 #pragma unroll
-  for (int jj = SPT - 1; jj >= 0; jj--) {
-    cum += gs[jj];
-    dchi[jj] = cum;
+  for (int i = 0; i < SPT; i++) {
+    cum += gs[i];
+    dchi[SPT - 1 - i] = cum;
   }
 }
 
@@ -2475,7 +2591,7 @@ template <typename R, int SPT>
 __device__ inline void rot_chi_adj(const R* gam, R ngp, R* gd, const RotRow<R>* __restrict__ rot_tab, int rot_states,
                                    double rot_fc, double dt, int N, int n0) {
   const int tid = threadIdx.x, nth = blockDim.x, lane = tid & 63, wave = tid >> 6, nwv = nth >> 6;
-  constexpr int G = sizeof(R) == 4 ? ROT_G32 : ROT_G64;
+  constexpr int G = sizeof(R) == 4 ? ROT_G32 : ROT_ADJ_G64;
   __shared__ R adj_wsr[16];
   __shared__ cplx<R> adj_ws[2][G][16];
   const R dtr = (R)dt, fc = (R)rot_fc;
@@ -2729,7 +2845,7 @@ __global__ __launch_bounds__(1024) void f_source(const cplx<T>* __restrict__ er,
     R drive[SPT];
 #pragma unroll
     for (int j = 0; j < SPT; j++) drive[j] = e[j] * e[j];
-    rot_chi<R, SPT>(drive, ngp, dchi, rot_tab, rot_states, rot_fc, dt, N, a0);
+    rot_chi<R, SPT>(drive, ngp, dchi, rot_tab, rot_states, rot_fc, dt);
   }
 
   // 3. Kerr chi = ng chi3/nref E^2 (uppe.cl:132-151), P = chi E, J_p = ne E, packed as P + i J_p
@@ -3052,7 +3168,7 @@ __global__ __launch_bounds__(1024) void f_source_env(const cplx<T>* __restrict__
     R drive[SPT];
 #pragma unroll
     for (int j = 0; j < SPT; j++) drive[j] = R(0.5) * (e[j].re * e[j].re + e[j].im * e[j].im);
-    rot_chi<R, SPT>(drive, ngp, dchi, rot_tab, rot_states, rot_fc, dt, N, a0);
+    rot_chi<R, SPT>(drive, ngp, dchi, rot_tab, rot_states, rot_fc, dt);
   }
 
   // chi = rotator + 0.75 n_g chi3 |E|^2 (paraxial.cl:112-131), P = chi E, Q = n_e (|A|^2/4 - 1) A (:99-110);
@@ -3363,7 +3479,7 @@ __global__ __launch_bounds__(1024) void f_source_adj_ion(const cplx<T>* __restri
       drive[j] = em * em;
       dchi[j] = T(0);
     }
-    rot_chi<T, SPT>(drive, (T)ngp, dchi, rot_tab, rot_states, rot_fc, dt, N, a0m);
+    rot_chi<T, SPT>(drive, (T)ngp, dchi, rot_tab, rot_states, rot_fc, dt);
     __syncthreads();  // every thread has read its R' samples from the second strip
 #pragma unroll
     for (int j = 0; j < SPT; j++) Z2[lds_swz<T>(a0m + j)] = cmk(dchi[j], T(0));
@@ -5717,33 +5833,61 @@ void fused_destroy(uppe_handle* h) {
   h->fused = nullptr;
 }
 
-template <typename T>
-static void rot_rows(uppe_handle* h, FusedState* s) {
-  // the source kernel's launch shape: nth threads, SPT samples each
-  const int N = h->nt, nth = std::max(std::min(N, 64), N / 4), spt = N / nth;
+template <typename T, int SPT>
+static void rot_upload(uppe_handle* h, FusedState* s) {
   const int n = h->rot_states - 2;
   std::vector<RotRow<T>> rows((size_t)n);
+  const int np = (n + rot_group<T>() - 1) / rot_group<T>() * rot_group<T>();  // whole groups: rows of zeros
+  std::vector<RotFwd<T, SPT>> fwd((size_t)np, RotFwd<T, SPT>());
+  std::vector<cplx<T>> pows((size_t)np * ROT_POW, cplx<T>{T(0), T(0)});
   for (int i = 0; i < n; i++) {
     const int sj = i + 2;
     const double wr = h->rot_wdt[2 * sj], wi = h->rot_wdt[2 * sj + 1];
     // E^k = exp(i k W dt / 2) for the complex W dt = wr + i wi (rotations.cl:107)
-    auto epow = [&](double k) {
-      const double mag = std::exp(-0.5 * wi * k);
-      return cplx<T>{(T)(mag * std::cos(0.5 * wr * k)), (T)(mag * std::sin(0.5 * wr * k))};
-    };
+    auto epow64 = [&](double k) { return std::polar(std::exp(-0.5 * wi * k), 0.5 * wr * k); };
+    auto narrow = [](std::complex<double> v) { return cplx<T>{(T)v.real(), (T)v.imag()}; };
+    const double c = h->rot_tjj[sj] * (2.0 * sj * (sj - 1) / (15.0 * (2 * sj - 1))) * 2.0 * h->rot_dalpha;
     RotRow<T>& r = rows[(size_t)i];
     r.wr64 = wr;
     r.wi64 = wi;
-    r.c = (T)(h->rot_tjj[sj] * (2.0 * sj * (sj - 1) / (15.0 * (2 * sj - 1))) * 2.0 * h->rot_dalpha);
+    r.c = (T)c;
     r.wr = (T)wr;
     r.wi = (T)wi;
     r.pad = T(0);
-    r.e[0] = epow(1.0);
-    r.e[1] = epow(2.0);
-    for (int b = 0; b < ROT_NB; b++) r.e[2 + b] = epow(2.0 * spt * (double)(1 << b));
+    r.e[0] = narrow(epow64(1.0));
+    r.e[1] = narrow(epow64(2.0));
+    for (int b = 0; b < ROT_NB; b++) r.e[2 + b] = narrow(epow64(2.0 * SPT * (double)(1 << b)));
+    RotFwd<T, SPT>& f = fwd[(size_t)i];
+    const std::complex<double> w(wr, wi);
+    f.k[0] = T(0);
+    for (int m = 0; m < SPT; m++) {
+      const std::complex<double> b = c * w * std::conj(epow64(2.0 * m));
+      f.e[m] = narrow(epow64(2.0 * m + 1.0));
+      f.b[m] = narrow(b);
+      for (int l = 0; l < m; l++) f.k[m * (m - 1) / 2 + l] = (T)std::real(epow64(2.0 * l + 1.0) * b);
+    }
+    for (int l = 0; l < 64; l++) pows[(size_t)i * ROT_POW + l] = narrow(epow64(2.0 * SPT * l));
+    for (int v = 0; v < 16; v++) pows[(size_t)i * ROT_POW + 64 + v] = narrow(epow64(2.0 * SPT * 64 * v));
   }
-  UPPE_HIP(hipMalloc(&s->rot_tab, sizeof(RotRow<T>) * (size_t)n));
-  UPPE_HIP(hipMemcpy(s->rot_tab, rows.data(), sizeof(RotRow<T>) * (size_t)n, hipMemcpyHostToDevice));
+  const size_t nb[3] = {sizeof(rows[0]) * n, sizeof(fwd[0]) * np, sizeof(pows[0]) * pows.size()};
+  UPPE_HIP(hipMalloc(&s->rot_tab, nb[0] + nb[1] + nb[2]));
+  char* d = static_cast<char*>(s->rot_tab);
+  UPPE_HIP(hipMemcpy(d, rows.data(), nb[0], hipMemcpyHostToDevice));
+  UPPE_HIP(hipMemcpy(d + nb[0], fwd.data(), nb[1], hipMemcpyHostToDevice));
+  UPPE_HIP(hipMemcpy(d + nb[0] + nb[1], pows.data(), nb[2], hipMemcpyHostToDevice));
+}
+
+template <typename T>
+static void rot_rows(uppe_handle* h, FusedState* s) {
+  // the launch shape of the source kernels that take a rotator: nth threads, N / nth samples each
+  const int N = h->nt, nth = std::max(std::min(N, 64), std::min(N / 4, 1024));
+  switch (N / nth) {
+    case 1: return rot_upload<T, 1>(h, s);
+    case 2: return rot_upload<T, 2>(h, s);
+    case 4: return rot_upload<T, 4>(h, s);
+    case 8: return rot_upload<T, 8>(h, s);
+  }
+  throw Error{UPPE_ERR_UNSUPPORTED, "rotator: unsupported Nt"};
 }
 
 void fused_set_rotator(uppe_handle* h) {
