@@ -440,7 +440,11 @@ __device__ inline cplx<float> linear_factor<float>(double phs, float ki, double 
 // ---------------------------------------------------------------------------------------------------
 // GEMM with fused prologue / epilogue:  out[M][2 nwp] = A[M][K] . B[K][2 nwp]
 // ---------------------------------------------------------------------------------------------------
-template <typename T, int PRO, int EPI>
+// RB rows per thread: 64-row tiles (4), and 16-row ones (1) for the one-off transforms at the ends of a run, whose grid
+// of 64-row tiles leaves a CU no second workgroup to hide its loads behind. A tile's next operands are requested ahead
+// of the products. Every RB sums a row in the same order. With both, us per launch, set-up / read-out: FP32 513 x 128
+// 19.1 / 19.9 -> 7.7 / 8.7, 1025 x 512 73 / 73 -> 35 / 41.
+template <typename T, int PRO, int EPI, int RB = 4>
 __global__ __launch_bounds__(256) void f_gemm(const T* __restrict__ A, const cplx<T>* __restrict__ B,
                                               cplx<T>* __restrict__ out, int M, int K, int nwp,
                                               const double* __restrict__ phs, const cplx<T>* __restrict__ kzc,
@@ -450,11 +454,12 @@ __global__ __launch_bounds__(256) void f_gemm(const T* __restrict__ A, const cpl
                                               StepState* __restrict__ st, unsigned long long* __restrict__ qmax,
                                               unsigned long long* __restrict__ qmax_next, int stage, double zfix,
                                               double qbfix, int f1fix) {
-  __shared__ T As[BK][BM + 1];
+  constexpr int BR = 16 * RB;
+  __shared__ T As[BK][BR + 1];
   __shared__ T Bs[BK][BN];
   __shared__ double red[8];
   const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int row0 = blockIdx.y * BM, col0 = blockIdx.x * BN;
+  const int row0 = blockIdx.y * BR, col0 = blockIdx.x * BN;
   double zph = zfix, cu = 0.0, dz = 0.0, qb = sizeof(T) == 4 ? qbfix : 0.0;
   int f1r = f1fix, rb_end = 0;
   if (st) {
@@ -470,52 +475,74 @@ __global__ __launch_bounds__(256) void f_gemm(const T* __restrict__ A, const cpl
       rb_end = sp.rb_end;
     }
   }
-  T acc[4][4];
+  T acc[RB][4];
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < RB; i++)
 #pragma unroll
     for (int j = 0; j < 4; j++) acc[i][j] = T(0);
 
-  for (int k0 = 0; k0 < K; k0 += BK) {
+  T ra[RB], rc[2];
+  cplx<T> rv[2], rk[2], rz[2];
+  double rp[2];
+  auto request = [&](int k0) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      int e = tid + 256 * i, r = e >> 4, kk = e & 15, gr = row0 + r, gk = k0 + kk;
-      As[kk][r] = (gr < M && gk < K) ? A[(long)gr * K + gk] : T(0);
+    for (int i = 0; i < RB; i++) {
+      const int e = tid + 256 * i, gr = row0 + (e >> 4), gk = k0 + (e & 15);
+      ra[i] = (gr < M && gk < K) ? A[(long)gr * K + gk] : T(0);
     }
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      int e = tid + 256 * i, kk = e >> 5, cf = e & 31, gk = k0 + kk, f = (col0 >> 1) + cf;
-      cplx<T> v = cmk(T(0), T(0));
+      const int e = tid + 256 * i, gk = k0 + (e >> 5), f = (col0 >> 1) + (e & 31);
+      rv[i] = rk[i] = cmk(T(0), T(0));
+      rz[i] = cmk(T(1), T(0));
+      rp[i] = 0.0;
+      rc[i] = T(1);
       if (gk < K) {
-        long idx = (long)gk * nwp + f;
-        v = B[idx];
-        if (pro_stage(PRO)) {
-          if (stage > 1) {
-            cplx<T> kp = kprev[idx];
-            T c = (T)cu;
-            v = cscale(cmk(v.re + c * kp.re, v.im + c * kp.im), cond[f]);
-          }
-          cplx<T> kz = kzc[idx];
-          v = cmul(linear_factor<T>(phs[idx], kz.im, zph, col_ref(f, f1r, zph, qb, 0).za, +1), v);
-          if (PRO == PRO_STAGE) v = cmul(cmk(-kz.im, kz.re), v);  // E = i kz A
-        } else if (PRO == PRO_FINISH) {
-          cplx<T> kz = kzc[idx];
-          v = cmul(linear_factor<T>(phs[idx], kz.im, zph, col_ref(f, f1r, zph, qb, 0).za, +1), v);
+        const long idx = (long)gk * nwp + f;
+        rv[i] = B[idx];
+        if (PRO != PRO_NONE) {
+          rz[i] = kzc[idx];
+          rp[i] = phs[idx];
+        }
+        if (pro_stage(PRO) && stage > 1) {
+          rk[i] = kprev[idx];
+          rc[i] = cond[f];
         }
       }
+    }
+  };
+  request(0);
+  for (int k0 = 0; k0 < K; k0 += BK) {
+#pragma unroll
+    for (int i = 0; i < RB; i++) {
+      const int e = tid + 256 * i;
+      As[e & 15][e >> 4] = ra[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int e = tid + 256 * i, kk = e >> 5, cf = e & 31, f = (col0 >> 1) + cf;
+      cplx<T> v = rv[i];
+      if (pro_stage(PRO) && stage > 1) {
+        const T c = (T)cu;
+        v = cscale(cmk(v.re + c * rk[i].re, v.im + c * rk[i].im), rc[i]);
+      }
+      if (PRO != PRO_NONE)
+        v = cmul(linear_factor<T>(rp[i], rz[i].im, zph, col_ref(f, f1r, zph, qb, 0).za, +1), v);
+      if (PRO == PRO_STAGE) v = cmul(cmk(-rz[i].im, rz[i].re), v);  // E = i kz A
       Bs[kk][2 * cf] = v.re;
       Bs[kk][2 * cf + 1] = v.im;
     }
     __syncthreads();
+    if (k0 + BK < K) request(k0 + BK);
 #pragma unroll
     for (int kk = 0; kk < BK; kk++) {
-      T a[4], b[4];
+      T a[RB], b[4];
 #pragma unroll
-      for (int i = 0; i < 4; i++) a[i] = As[kk][ty * 4 + i];
+      for (int i = 0; i < RB; i++) a[i] = As[kk][ty * RB + i];
 #pragma unroll
       for (int j = 0; j < 4; j++) b[j] = Bs[kk][tx * 4 + j];
 #pragma unroll
-      for (int i = 0; i < 4; i++)
+      for (int i = 0; i < RB; i++)
 #pragma unroll
         for (int j = 0; j < 4; j++) acc[i][j] += a[i] * b[j];
     }
@@ -525,8 +552,8 @@ __global__ __launch_bounds__(256) void f_gemm(const T* __restrict__ A, const cpl
   double loc = (EPI == EPI_STAGE && stage == 4) ? 0.0 : INFINITY;
   bool nan = false;
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int r = row0 + ty * 4 + i;
+  for (int i = 0; i < RB; i++) {
+    const int r = row0 + ty * RB + i;
     if (r >= M) continue;
 #pragma unroll
     for (int jj = 0; jj < 2; jj++) {
@@ -3523,32 +3550,38 @@ __global__ void f_fill_zero(unsigned long long* p, long n) {
 }
 
 // max |q| over the state (set_field)
+// max|q| over P rows of columns [f_all, nwp) into all and over columns [f_from, nwp) into part (f_all <= f_from): a
+// block takes whole rows and adds one value to each word (a word takes an atomic every 12 ns: one per wavefront of 256
+// blocks cost 13 us, whatever the field)
 template <typename T>
-__global__ void f_qmax(const cplx<T>* q, long n, unsigned long long* out) {
-  double m = 0.0;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    cplx<T> v = q[i];
-    m = fmax(m, sqrt((double)v.re * v.re + (double)v.im * v.im));
-  }
-  for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
-  if ((threadIdx.x & 63) == 0) atomicMax(out, dbits(m));
-}
-
-// max |q| over complex columns [f_from, nwp) of every row
-template <typename T>
-__global__ void f_qmax_cols(const cplx<T>* q, long P, int nwp, int f_from, unsigned long long* out) {
-  const int w = nwp - f_from;
-  double m = 0.0;
-  if (w > 0)
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < P * w; i += (long)gridDim.x * blockDim.x) {
-      cplx<T> v = q[(i / w) * nwp + f_from + (i % w)];
-      m = fmax(m, sqrt((double)v.re * v.re + (double)v.im * v.im));
+__global__ __launch_bounds__(256) void f_qmax(const cplx<T>* q, long P, int nwp, int f_all, int f_from,
+                                              unsigned long long* all, unsigned long long* part) {
+  __shared__ double red[2][4];
+  double ma = 0.0, mp = 0.0;  // the largest |q|^2: its root is the largest root
+  for (long r = blockIdx.x; r < P; r += gridDim.x)
+    for (int f = f_all + threadIdx.x; f < nwp; f += 256) {
+      const cplx<T> v = q[r * nwp + f];
+      const double m = (double)v.re * v.re + (double)v.im * v.im;
+      ma = fmax(ma, m);
+      if (f >= f_from) mp = fmax(mp, m);
     }
-  for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
-  if ((threadIdx.x & 63) == 0) atomicMax(out, dbits(m));
+  for (int o = 32; o > 0; o >>= 1) {
+    ma = fmax(ma, __shfl_xor(ma, o));
+    mp = fmax(mp, __shfl_xor(mp, o));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = ma;
+    red[1][threadIdx.x >> 6] = mp;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    const double* m = red[threadIdx.x];
+    const double v = sqrt(fmax(fmax(m[0], m[1]), fmax(m[2], m[3])));
+    unsigned long long* out = threadIdx.x == 0 ? all : part;
+    if (out && v > 0.0) atomicMax(out, dbits(v));
+  }
 }
 
-// host layout (nw, P) complex128 -> [P][nwp] complex T (zero padding)
 template <typename T>
 __global__ void f_from_host(const double* src, cplx<T>* dst, int nw, long P, int nwp) {
   long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
@@ -3883,7 +3916,7 @@ static bool wave_source_forced() {
 }
 
 // the stepping source kernel (no diagnostics, no rotator) for Nt = 2^LG, where the block of Nt / S threads fits
-// 64..1024; otherwise the kernel for any Nt. FP64 at 128 strips, launch 15.4 -> 11 us (2048 samples, O2), 8.0 -> 6.4
+// 64..1024; otherwise the kernel for any Nt. FP64 at 128 strips, launch 15.4 -> 12.0 us (2048 samples, O2), 8.0 -> 6.4
 // (1024, Kerr), the rate as one exponential and the twiddles requested early among them.
 template <typename T, int S, int LG>
 constexpr auto source_fixed() {
@@ -4221,24 +4254,35 @@ struct Fused {
     UPPE_HIP(hipStreamSynchronize(h->stream));
   }
 
+  // max|q| over the columns the r2k direction never updates into qmax[2], and over all columns into all
+  static void qmax_launch(uppe_handle* h, FusedState* s, int f_all, unsigned long long* all) {
+    launchf(h, UPPE_KC_REDUCE, f_qmax<T>, dim3((unsigned)std::min(h->P, h->P > 2048 ? 512L : 128L)), dim3(256), 0,
+            (const C*)s->q, h->P, s->nwp, f_all, s->f1, all, s->qmax + 2);
+  }
+
   static void static_qmax(uppe_handle* h, FusedState* s) {
     UPPE_HIP(hipMemsetAsync(s->qmax + 2, 0, sizeof(unsigned long long), h->stream));
-    launchf(h, UPPE_KC_REDUCE, f_qmax_cols<T>, dim3(256), dim3(kBlock), 0, (const C*)s->q, h->P, s->nwp, s->f1,
-            s->qmax + 2);
+    qmax_launch(h, s, s->f1, nullptr);
     UPPE_HIP(hipStreamSynchronize(h->stream));
   }
 
   // SIMT contraction (the one-off transforms of set_field/finish): one launch per azimuthal mode m over the rows
   // r N2 + m, with that mode's operator
-  static void gemm_r2k_plain(uppe_handle* h, FusedState* s, const C* in, C* out) {
-    dim3 grid(2 * s->nwp / BN, (h->nk + BM - 1) / BM);
-    const int row = h->n2 * s->nwp;
-    for (int m = 0; m < h->n2; m++)
-      launchf(h, UPPE_KC_HANKEL, f_gemm<T, PRO_NONE, EPI_NONE>, grid, dim3(256), 0,
-              (const T*)s->Hf + (size_t)m * h->n1 * h->nk, in + (long)m * s->nwp, out + (long)m * s->nwp, h->nk,
-              h->n1, row, (const double*)nullptr, (const C*)nullptr, (const T*)nullptr, (C*)nullptr,
-              (const C*)nullptr, (C*)nullptr, (C*)nullptr, (C*)nullptr, (StepState*)nullptr,
-              (unsigned long long*)nullptr, (unsigned long long*)nullptr, 0, 0.0, 0.0, 0);
+  // a transform outside the steps: every azimuthal mode's out = A in. 16-row tiles while 64-row ones are fewer than
+  // four per CU (FP32) or one (FP64, where every row tile repeats the prologue's double sines and exponentials)
+  template <int PRO>
+  static void gemm_once(uppe_handle* h, FusedState* s, const T* A, const C* in, C* out, int M, int K, double z,
+                        double qbase, int f1) {
+    const int gx = 2 * s->nwp / BN, row = h->n2 * s->nwp;
+    const bool low = (long)gx * ((M + BM - 1) / BM) < (sizeof(T) == 4 ? 4L : 1L) * s->n_cu;
+    const dim3 grid(gx, low ? (M + 15) / 16 : (M + BM - 1) / BM);
+    for (int m = 0; m < h->n2; m++) {
+      const long o = (long)m * s->nwp;
+      launchf(h, UPPE_KC_HANKEL, low ? f_gemm<T, PRO, EPI_NONE, 1> : f_gemm<T, PRO, EPI_NONE>, grid, dim3(256), 0,
+              A + (size_t)m * M * K, in + o, out + o, M, K, row, (const double*)s->phs + o, (const C*)s->kzc + o,
+              (const T*)s->cond, (C*)nullptr, (const C*)nullptr, (C*)nullptr, (C*)nullptr, (C*)nullptr,
+              (StepState*)nullptr, (unsigned long long*)nullptr, (unsigned long long*)nullptr, 0, z, qbase, f1);
+    }
   }
 
   // the DFT over the azimuthal points of every (r, f < ncols) with exponent sign `sign`, scaled by sc (default:
@@ -4695,12 +4739,10 @@ struct Fused {
       tpass<PRO_NONE, EPI_NONE>(h, s, 2, (const C*)s->er, (C*)s->q, h->nw, -1, nullptr, 0, 0.0, nullptr);
     } else {
       azim(h, s, (C*)s->er, h->nw, -1);  // FFT_axis2 first (grid_tools.py:308-316)
-      gemm_r2k_plain(h, s, (const C*)s->er, (C*)s->q);
+      gemm_once<PRO_NONE>(h, s, (const T*)s->Hf, (const C*)s->er, (C*)s->q, h->nk, h->n1, 0.0, 0.0, 0);
     }
     UPPE_HIP(hipMemsetAsync(s->qmax, 0, sizeof(unsigned long long) * kQW, h->stream));
-    launchf(h, UPPE_KC_REDUCE, f_qmax<T>, dim3(256), dim3(kBlock), 0, (const C*)s->q, P * s->nwp, s->qmax);
-    launchf(h, UPPE_KC_REDUCE, f_qmax_cols<T>, dim3(256), dim3(kBlock), 0, (const C*)s->q, P, s->nwp, s->f1,
-            s->qmax + 2);
+    qmax_launch(h, s, 0, s->qmax);
     UPPE_HIP(hipStreamSynchronize(h->stream));
   }
 
@@ -5060,22 +5102,14 @@ struct Fused {
       tpass<PRO_FINISH, EPI_NONE>(h, s, 2, (const C*)s->q, (C*)s->er, h->nw, +1, nullptr, 0, z_total, nullptr);
       tpass<PRO_NONE, EPI_NONE>(h, s, 1, (const C*)s->er, (C*)s->er, h->nw, +1, nullptr, 0, z_total, nullptr);
     } else {
-      dim3 g_k2r(2 * s->nwp / BN, (h->n1 + BM - 1) / BM);
-      const int row = h->n2 * s->nwp;
-      for (int m = 0; m < h->n2; m++) {
-        const long o = (long)m * s->nwp;
-        launchf(h, UPPE_KC_HANKEL, f_gemm<T, PRO_FINISH, EPI_NONE>, g_k2r, dim3(256), 0,
-                (const T*)s->Hb + (size_t)m * h->n1 * h->nk, (const C*)s->q + o, (C*)s->er + o, h->n1, h->nk, row,
-                (const double*)s->phs + o, (const C*)s->kzc + o, (const T*)s->cond, (C*)nullptr, (const C*)nullptr,
-                (C*)nullptr, (C*)nullptr, (C*)nullptr, (StepState*)nullptr, (unsigned long long*)nullptr,
-                (unsigned long long*)nullptr, 0, z_total, s->qbase, s->f1);
-      }
+      gemm_once<PRO_FINISH>(h, s, (const T*)s->Hb, (const C*)s->q, (C*)s->er, h->n1, h->nk, z_total, s->qbase, s->f1);
       azim(h, s, (C*)s->er, h->nw, +1);
     }
-    if (h->paraxial) {
+    const bool diag = j_r || chi_t || ne_t;  // the field alone needs no source
+    if (diag && h->paraxial) {
       // the envelope source takes A itself (paraxial_kernel.py:243-245)
       source(h, s, (const C*)s->er, (C*)s->jr, true, nullptr);
-    } else {
+    } else if (diag) {
       UPPE_HIP(hipMemcpyAsync(s->k1, s->er, sizeof(C) * n, hipMemcpyDeviceToDevice, h->stream));
       launchf(h, UPPE_KC_POINT, f_vp_to_e<T>, dim3(grid_for(n)), dim3(kBlock), 0, (C*)s->k1, (const C*)s->kzc, n);
       source(h, s, (const C*)s->k1, (C*)s->jr, true, nullptr);
@@ -5096,9 +5130,9 @@ struct Fused {
     if (j_r) out_c(s->jr, j_r);
     if (chi_t) out_t(s->chi_t, chi_t);
     if (ne_t) out_t(s->ne_t, ne_t);
+    // the diagnostics leave k1 holding the r-space field: clear it so the next run starts from zero stage buffers
+    if (diag) UPPE_HIP(hipMemsetAsync(s->k1, 0, sizeof(C) * n, h->stream));
     UPPE_HIP(hipStreamSynchronize(h->stream));
-    // finish leaves k1 holding the r-space field: clear it so the next run starts from zero stage buffers
-    UPPE_HIP(hipMemset(s->k1, 0, sizeof(C) * n));
   }
 
   static void get_state(uppe_handle* h, FusedState* s, double* q) {
