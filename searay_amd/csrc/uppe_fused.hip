@@ -5911,14 +5911,25 @@ static void rot_upload(uppe_handle* h, FusedState* s) {
     RotFwd<T, SPT>& f = fwd[(size_t)i];
     const std::complex<double> w(wr, wi);
     f.k[0] = T(0);
+    std::complex<double> odd[SPT];  // E^(2m+1)
     for (int m = 0; m < SPT; m++) {
       const std::complex<double> b = c * w * std::conj(epow64(2.0 * m));
-      f.e[m] = narrow(epow64(2.0 * m + 1.0));
+      odd[m] = epow64(2.0 * m + 1.0);
+      f.e[m] = narrow(odd[m]);
       f.b[m] = narrow(b);
-      for (int l = 0; l < m; l++) f.k[m * (m - 1) / 2 + l] = (T)std::real(epow64(2.0 * l + 1.0) * b);
+      for (int l = 0; l < m; l++) f.k[m * (m - 1) / 2 + l] = (T)std::real(odd[l] * b);
     }
-    for (int l = 0; l < 64; l++) pows[(size_t)i * ROT_POW + l] = narrow(epow64(2.0 * SPT * l));
-    for (int v = 0; v < 16; v++) pows[(size_t)i * ROT_POW + 64 + v] = narrow(epow64(2.0 * SPT * 64 * v));
+    // the powers as products of two (an exponential, sine and cosine each would double the handle's set-up)
+    auto products = [&](cplx<T>* out, int count, int low, double step) {
+      std::complex<double> lo[8];
+      for (int l = 0; l < low; l++) lo[l] = epow64(step * l);
+      for (int l0 = 0; l0 < count; l0 += low) {
+        const std::complex<double> hi = epow64(step * l0);
+        for (int l = 0; l < low; l++) out[l0 + l] = narrow(hi * lo[l]);
+      }
+    };
+    products(&pows[(size_t)i * ROT_POW], 64, 8, 2.0 * SPT);
+    products(&pows[(size_t)i * ROT_POW + 64], 16, 4, 2.0 * SPT * 64);
   }
   const size_t nb[3] = {sizeof(rows[0]) * n, sizeof(fwd[0]) * np, sizeof(pows[0]) * pows.size()};
   UPPE_HIP(hipMalloc(&s->rot_tab, nb[0] + nb[1] + nb[2]));
