@@ -1035,10 +1035,11 @@ __device__ inline void hankel_tile(
     }
     __syncthreads();
 
-    // ---- MFMA main loop over the chunk's contraction chunks (global indices: the ring prefetches across chunks). A
-    // tile of one MFMA column tile (all but the grid's last, unless wide) reads the slab operands of a whole ring before
-    // its products and tests no column count between them; read one product at a time, each product waited for its
-    // operand (FP32, us per launch: 513 x 128 adjoint r2k 7.7 -> 6.7, k2r 6.5 -> 5.5; 1025 x 512 r2k 23.2 -> 20.4).
+    // ---- MFMA main loop over the chunk's contraction chunks (global indices: the ring prefetches across chunks). With
+    // one row tile per wave, a tile of one MFMA column tile (all but the grid's last, unless wide) reads the slab
+    // operands of a whole ring before its products and tests no column count between them; read one product at a time,
+    // each product waited for its operand (FP32, us per launch: 513 x 128 adjoint r2k 7.7 -> 6.7, k2r 6.5 -> 5.5; 1025 x
+    // 512 r2k 23.2 -> 20.4). With two row tiles the second loop would spill registers.
     auto main_loop = [&](auto one) {
       constexpr int NC = decltype(one)::value ? 1 : CT;    // MFMA column tiles
       constexpr int PD = decltype(one)::value ? RING : 1;  // chunks whose slab operands are read together
@@ -1111,10 +1112,11 @@ __device__ inline void hankel_tile(
         }
       }
     };
-    if (nmt == 1)
-      main_loop(std::true_type());
-    else
+    if (RT == 1 && nmt == 1) {
+      if constexpr (RT == 1) main_loop(std::true_type());
+    } else {
       main_loop(std::false_type());
+    }
   }  // contraction chunks
   __syncthreads();  // B slab no longer needed: reuse LDS for the output tile
 
