@@ -60,21 +60,16 @@ class AnalyticBox:
             np.save(basename + '_' + self.name + '_' + suffix, arr)
 
     def GetRelDensityPlanes(self, xp, zs):
-        '''GetRelDensity of the points xp (N1, N2, 8) moved to each z of zs, in one evaluation of the density lambda:
-        an array (len(zs), N1, N2), or None where the lambda does not map positions to densities of their shape (one
-        that returns a plain number, or changes its arguments in place).'''
-        zs = np.asarray(zs, dtype=float)
-        shape = zs.shape + xp.shape[:2]
-
-        def planes(a):
-            return np.broadcast_to(a, shape)
+        '''GetRelDensity of the points xp (N1, N2, 8) moved to each z of zs in turn (xp[..., 3] is written): the density
+        lambda gets one plane at a time, as there, with r2 formed once. r2 is handed out as a fresh copy, and a lambda
+        that changes x or y makes the planes after it stale.'''
+        x = xp[..., 1]
+        y = xp[..., 2]
+        z = xp[..., 3]
         r2 = np.einsum('...i,...i', xp[..., 1:3], xp[..., 1:3])
-        try:
-            dens = np.asarray(self.vol_dict['density lambda'](planes(xp[..., 1]), planes(xp[..., 2]),
-                                                              planes(zs[:, None, None]), planes(r2)), dtype=float)
-        except (ValueError, TypeError, IndexError):
-            return None
-        return dens if dens.shape == shape else None
+        for zk in zs:
+            z.fill(zk)
+            yield self.vol_dict['density lambda'](x, y, z, r2.copy())
 
     def GetRelDensity(self, xp):
         x = xp[..., 1]
