@@ -5194,7 +5194,7 @@ struct FusedBatch {
   std::vector<MemberSlots> slots;  // per member (addresses handed to the member states)
   std::vector<int> group_of, slot_of;
   std::vector<BatchRun> runs;      // runs of the last advance
-  // tuned launch shapes by run: (group, first, count, f1) -> plans and samples per thread
+  // tuned launch shapes by run: (group, first, count, f1, shared tables, rotator) -> plans and samples per thread
   std::vector<std::pair<std::vector<long>, BatchRun>> tuned;
   bool autotune = true;
   // HIP graph of graph_steps steps of every run (0: launch step by step), launched on `main`; the runs'
@@ -5743,7 +5743,7 @@ void fused_batch_advance(uppe_batch* b, const uppe_step_control* c, int* steps_o
         if (!(sm->tab_fp == h0->fused->tab_fp)) r.share &= ~2;
       }
       if (fb->autotune) {
-        const std::vector<long> key = {g, r.first, r.count, h0->fused->f1, r.share};
+        const std::vector<long> key = {g, r.first, r.count, h0->fused->f1, r.share, h0->rot_states > 2};
         auto it = std::find_if(fb->tuned.begin(), fb->tuned.end(), [&](const auto& e) { return e.first == key; });
         if (it != fb->tuned.end()) {
           const bool known = r.known;
@@ -5958,6 +5958,9 @@ void fused_set_rotator(uppe_handle* h) {
   FusedState* s = h->fused;
   if (s->rot_tab) UPPE_HIP(hipFree(s->rot_tab));
   s->rot_tab = nullptr;
+  // the source's launch shape depends on whether there is a rotator: the next run chooses it again
+  s->spt = 0;
+  s->tuned_f1 = -1;
   if (h->rot_states < 3) return;
   if (is_fp64(h))
     rot_rows<double>(h, s);
