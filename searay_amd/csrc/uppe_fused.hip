@@ -1316,7 +1316,7 @@ struct XArgs {
 // How a tile's complex columns lie in the 16 real columns of a matrix product. X_WIDE: 8 complex columns, re and im
 // side by side. X_HALF: up to 4 in the lower 8 columns, the upper ones unused. X_PACK (BF16x3): up to 4, their hi
 // halves in the lower 8 columns and lo halves in the upper 8, so that two products (A_hi and A_lo with the packed
-// tile) give all four partial products.
+// tile) give all four partial products; the other layouts form the same four.
 enum { X_WIDE = 0, X_HALF = 1, X_PACK = 2 };
 
 // LDS slab of a contraction's B operand, kp rows (k) of 16 real columns. BF16x3: columns of k-contiguous halves
@@ -1393,7 +1393,10 @@ struct XRing {
 };
 
 // acc += A . slab over all chunks (16 or 32 rows of the slab each); ring holds the first chunks' fragments. The slab
-// operands of a whole ring are read before its products.
+// operands of a whole ring are read before its products. BF16x3 sums the products with the slab's lo halves apart in
+// every layout: a packed tile has them in its upper columns, the others in a second accumulator. The plans of a grid,
+// which autotuned batches choose by timing, then differ in no bit of the result; three products in one accumulator
+// took as long (2049 x 256 on 256 CUs, 11.91 and 11.93 ms per 100 steps).
 template <int CM, int RT, int LAY>
 __device__ __forceinline__ void x_contract(typename MfmaTraits<CM>::acc_t (&acc)[RT], XRing<CM, RT>& ring,
                                            const typename MfmaTraits<CM>::frag_t* __restrict__ hi,
@@ -1406,18 +1409,21 @@ __device__ __forceinline__ void x_contract(typename MfmaTraits<CM>::acc_t (&acc)
 #pragma unroll
   for (int r = 0; r < RT; r++) acc[r] = typename MfmaTraits<CM>::acc_t{0, 0, 0, 0};
   if (mt0 >= m16) return;  // a wave without rows
+  constexpr bool LO = CM == CM_BF16X3 && LAY != X_PACK;
+  typename MfmaTraits<CM>::acc_t low[LO ? RT : 1];
+#pragma unroll
+  for (int r = 0; r < (LO ? RT : 1); r++) low[r] = typename MfmaTraits<CM>::acc_t{0, 0, 0, 0};
   auto group = [&](int c0, auto whole) {
     constexpr bool W = decltype(whole)::value;  // all RING chunks are there
     if constexpr (CM == CM_BF16X3) {
-      constexpr bool P = LAY == X_PACK;
-      bf16x8 vh[RING], vl[P ? 1 : RING];
+      bf16x8 vh[RING], vl[LO ? RING : 1];
       const int ldb = kp + 8;
       const __bf16* bh = reinterpret_cast<const __bf16*>(slab) + col * ldb + c0 * 32 + 8 * quad;
 #pragma unroll
       for (int d = 0; d < RING; d++)
         if (W || c0 + d < nch) {
           vh[d] = *reinterpret_cast<const bf16x8*>(bh + d * 32);
-          if constexpr (!P) vl[d] = *reinterpret_cast<const bf16x8*>(bh + d * 32 + 16 * ldb);
+          if constexpr (LO) vl[d] = *reinterpret_cast<const bf16x8*>(bh + d * 32 + 16 * ldb);
         }
 #pragma unroll
       for (int d = 0; d < RING; d++)
@@ -1426,8 +1432,11 @@ __device__ __forceinline__ void x_contract(typename MfmaTraits<CM>::acc_t (&acc)
           for (int r = 0; r < RT; r++)
             if (mt0 + r < m16) {
               acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring.h[d][r], vh[d], acc[r], 0, 0, 0);
-              if constexpr (!P) acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring.h[d][r], vl[d], acc[r], 0, 0, 0);
               acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring.l[d][r], vh[d], acc[r], 0, 0, 0);
+              if constexpr (LO) {
+                low[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring.h[d][r], vl[d], low[r], 0, 0, 0);
+                low[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring.l[d][r], vl[d], low[r], 0, 0, 0);
+              }
             }
           ring.fetch(hi, lo, nch, m16, mt0, lane, c0 + d + RING, d);
         }
@@ -1459,6 +1468,10 @@ __device__ __forceinline__ void x_contract(typename MfmaTraits<CM>::acc_t (&acc)
   int c0 = 0;
   for (; c0 + RING <= nch; c0 += RING) group(c0, std::true_type());
   if (c0 < nch) group(c0, std::false_type());
+  if constexpr (LO) {
+#pragma unroll
+    for (int r = 0; r < RT; r++) acc[r] += low[r];
+  }
 }
 
 // A result tile leaves row rin(i) (i < 4) of real column lane % 16 in element i of a lane's accumulator. The two
