@@ -912,7 +912,6 @@ __device__ inline void hankel_tile(
   // slab is staged so their latency overlaps it
   using F = typename MfmaTraits<CM>::frag_t;
   constexpr int RING = (CM == CM_F64 || RT == 2) ? 2 : 4;
-  constexpr int rt_n = RT;  // 16-row tiles per wave (rw = 16 RT)
   const int mt0 = (row0 + wave * rw) / 16;  // first 16-row tile of this wave
   const int M16 = (M + 15) / 16;
   const int NCH = CM == CM_BF16X3 ? Kp / 32 : Kp / 16;  // contraction chunks
@@ -1039,10 +1038,16 @@ __device__ inline void hankel_tile(
     // one row tile per wave, a tile of one MFMA column tile (all but the grid's last, unless wide) reads the slab
     // operands of a whole ring before its products and tests no column count between them; read one product at a time,
     // each product waited for its operand (FP32, us per launch: 513 x 128 adjoint r2k 7.7 -> 6.7, k2r 6.5 -> 5.5; 1025 x
-    // 512 r2k 23.2 -> 20.4). With two row tiles the second loop would spill registers.
+    // 512 r2k 23.2 -> 20.4). With two row tiles per wave the operand rows come one by one: four at once cost FP64, which
+    // spills, half as much again (us per k2r launch: 2049 x 512 196 -> 122, 1025 x 1024 369 -> 226) and FP32 a twentieth
+    // (2049 x 512 50.3 -> 47.8). FP32 has the registers for a second loop with a chunk's four rows at once. It pays while
+    // the operator is small (us per k2r launch, one by one / at once: 4097 x 512 100 / 86; 2049 x 1024, whose operator is
+    // an XCD's L2, 190 / 200; 513 x 2048 198 / 203).
     auto main_loop = [&](auto one) {
-      constexpr int NC = decltype(one)::value ? 1 : CT;    // MFMA column tiles
-      constexpr int PD = decltype(one)::value ? RING : 1;  // chunks whose slab operands are read together
+      constexpr bool ONE = decltype(one)::value;
+      constexpr int NC = ONE ? 1 : CT;               // MFMA column tiles
+      constexpr int PD = ONE && RT == 1 ? RING : 1;  // chunks whose slab operands are read together
+      constexpr int JD = ONE || RT == 1 ? 4 : 1;     // and of a chunk's four operand rows (FP64, FP32)
       constexpr int KS = CM == CM_BF16X3 ? 32 : 16;        // slab rows of a chunk
       const int end = (kb + kcn) / KS;
       for (int c0 = kb / KS; c0 < end; c0 += RING) {
@@ -1079,41 +1084,46 @@ __device__ inline void hankel_tile(
             }
           } else {
             const T* bs = reinterpret_cast<const T*>(smem) + ((lane >> 4) - kb) * BW + (lane & 15);
-            T b[PD][4][NC];
 #pragma unroll
-            for (int p = 0; p < PD; p++)
-              if (c0 + d0 + p < end)
+            for (int j0 = 0; j0 < 4; j0 += JD) {
+              T b[PD][JD][NC];
 #pragma unroll
-                for (int j = 0; j < 4; j++)
+              for (int p = 0; p < PD; p++)
+                if (c0 + d0 + p < end)
 #pragma unroll
-                  for (int c = 0; c < NC; c++)
-                    b[p][j][c] = NC == 1 || c < nmt ? bs[((c0 + d0 + p) * 16 + 4 * j) * BW + c * 16] : T(0);
+                  for (int j = 0; j < JD; j++)
 #pragma unroll
-            for (int p = 0; p < PD; p++) {
-              const int d = d0 + p;
-              if (c0 + d >= end) break;
+                    for (int c = 0; c < NC; c++)
+                      b[p][j][c] = NC == 1 || c < nmt ? bs[((c0 + d0 + p) * 16 + 4 * (j0 + j)) * BW + c * 16] : T(0);
 #pragma unroll
-              for (int j = 0; j < 4; j++)
+              for (int p = 0; p < PD; p++) {
+                const int d = d0 + p;
+                if (c0 + d >= end) break;
 #pragma unroll
-                for (int r = 0; r < RT; r++) {
-                  if (mt0 + r >= M16) break;
+                for (int j = 0; j < JD; j++)
 #pragma unroll
-                  for (int c = 0; c < NC; c++) {
-                    if (NC > 1 && c >= nmt) break;
-                    if constexpr (CM == CM_F64)
-                      acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(ring_h[d][r][j], b[p][j][c], acc[r][c], 0, 0, 0);
-                    else
-                      acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(ring_h[d][r][j], b[p][j][c], acc[r][c], 0, 0, 0);
+                  for (int r = 0; r < RT; r++) {
+                    if (mt0 + r >= M16) break;
+#pragma unroll
+                    for (int c = 0; c < NC; c++) {
+                      if (NC > 1 && c >= nmt) break;
+                      const T av = ring_h[d][r][j0 + j], bv = b[p][j][c];
+                      if constexpr (CM == CM_F64)
+                        acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[r][c], 0, 0, 0);
+                      else
+                        acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc[r][c], 0, 0, 0);
+                    }
                   }
-                }
-              fetch_frag(c0 + d + RING, d);
+                if (j0 + JD == 4) fetch_frag(c0 + d + RING, d);
+              }
             }
           }
         }
       }
     };
-    if (RT == 1 && nmt == 1) {
-      if constexpr (RT == 1) main_loop(std::true_type());
+    constexpr bool two_loops = RT == 1 || CM == CM_F32;
+    if (two_loops && nmt == 1 && (RT == 1 || Kp <= 512)) {
+      if constexpr (two_loops) main_loop(std::true_type());
     } else {
       main_loop(std::false_type());
     }
