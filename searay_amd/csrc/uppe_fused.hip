@@ -1381,7 +1381,7 @@ __device__ __forceinline__ void x_put1(char* slab, int kp, int k, int cf, cplx<t
 // the operator's fragments of one contraction: a ring of RING chunks for the RT row tiles of a wave
 template <int CM, int RT>
 struct XRing {
-  static constexpr int RING = (CM == CM_F64 || RT >= 2) ? 2 : 4;
+  static constexpr int RING = CM == CM_F64 ? 2 : 4;
   using F = typename MfmaTraits<CM>::frag_t;
   F h[RING][RT], l[RING][CM == CM_BF16X3 ? RT : 1];
   __device__ __forceinline__ void fetch(const F* __restrict__ hi, const F* __restrict__ lo, int nch, int m16, int mt0,
@@ -3911,16 +3911,14 @@ static size_t x_lds(int cm, int kpf, int kpb) {
   return 2 * (cm == CM_F64 ? x_slab_bytes<CM_F64>(kp) : (cm == CM_F32 ? x_slab_bytes<CM_F32>(kp) : x_slab_bytes<CM_BF16X3>(kp)));
 }
 
-// exchange over nr radial cells in nl tiles of wn complex columns (4 or 8); wn = 0 in the result where no kernel
-// has the shape: wide tiles with more than 2 row tiles per wave in FP64, or more than one elsewhere, would spill
+// exchange over nr <= 256 radial cells in nl tiles of wn complex columns (4 or 8)
 static FusedState::XPlan x_shape(int cm, int nr, int wn) {
   FusedState::XPlan p;
   const int m16 = (nr + 15) / 16;
   p.nwv = std::min(x_max_waves(cm), m16);
   p.rt = (m16 + p.nwv - 1) / p.nwv;
-  if (p.rt == 3) p.rt = 4;
   p.wl = 8;
-  p.wn = p.rt > (cm == CM_F64 ? 4 : 2) || (wn > 4 && p.rt > (cm == CM_F64 ? 2 : 1)) ? 0 : wn;
+  p.wn = wn;
   return p;
 }
 
@@ -3929,18 +3927,13 @@ static FusedState::XPlan x_shape(int cm, int nr, int wn) {
 // that the operator, which every tile reads whole, is the larger cost. Measured, us per step, separate / 4 / 8
 // columns: BF16x3 Kerr 513 x 128 66 / 50 / 55, O2 2049 x 256 117 / 111 / 106; FP64 513 x 128 109 / 77 / 81,
 // O2 1025 x 128 201 / 173 / 169. Above 256 cells one tile's contractions hold a CU for longer than the separate
-// kernels, which split their rows over CUs, unless the grid has tiles for every CU (BF16x3 513 x 512 123 / 117;
-// FP64 2049 x 512 1486 / 680, 513 x 512 298 / 363); FP32 stays with them (513 x 512 194 / 230).
+// kernels, which split their rows over CUs (separate / 4 columns: BF16x3 129 x 512 116 / 124, 1025 x 512 165 / 203;
+// FP32 513 x 512 194 / 230; FP64 513 x 512 323 / 392, 1025 x 512 391 / 546, 2049 x 512 1016 / 1180).
 static FusedState::XPlan plan_exchange(int cm, int nr, int f1, int nw, int instances, int n_cu) {
   // SEARAY_UPPE_TILE_WIDTH pins the tiling of the separate contractions, so it asks for them
-  if (cm < 0 || nr > 512 || getenv("SEARAY_UPPE_TILE_WIDTH")) return FusedState::XPlan();
+  if (cm < 0 || nr > 256 || getenv("SEARAY_UPPE_TILE_WIDTH")) return FusedState::XPlan();
   const int nlt = (f1 + 3) / 4, lin = (std::max(0, nw - 4 * nlt) + 7) / 8;
-  const bool at_once = (long)(nlt + lin) * instances <= n_cu;
-  if (nr > 256) {
-    if (cm == CM_F32 || at_once != (cm == CM_BF16X3)) return FusedState::XPlan();
-    return x_shape(cm, nr, 4);
-  }
-  return x_shape(cm, nr, at_once ? 4 : 8);
+  return x_shape(cm, nr, (long)(nlt + lin) * instances <= n_cu ? 4 : 8);
 }
 
 template <typename T>
@@ -4588,7 +4581,7 @@ struct Fused {
     a.keep = keep;
     const int lin = std::max(0, (h->nw - a.nlt * pl.wn + pl.wl - 1) / pl.wl);
     const size_t shm = x_lds(CM, a.kpf, a.kpb);
-    if (pl.wn < 1 || 16 * pl.nwv * pl.rt < h->n1 || shm > kMaxLds)
+    if (pl.wn < 1 || pl.rt > (CM == CM_F64 ? 2 : 1) || 16 * pl.nwv * pl.rt < h->n1 || shm > kMaxLds)
       throw Error{UPPE_ERR_STATE, "exchange plan out of date"};
     // no linear tile has anything to do from stage 2 to 3, where the phase coordinate stands still, and in a launch
     // that ends with its slopes
@@ -4602,13 +4595,11 @@ struct Fused {
         UPPE_X(1, X_WIDE);
       else
         UPPE_X(1, half);
-    } else if (pl.rt == 2 && !wide) {
-      UPPE_X(2, half);
-    } else if constexpr (CM == CM_F64) {  // the shapes x_shape admits
+    } else if constexpr (CM == CM_F64) {  // 8 waves of up to two row tiles
       if (wide)
         UPPE_X(2, X_WIDE);
       else
-        UPPE_X(4, half);
+        UPPE_X(2, half);
     }
 #undef UPPE_X
   }
@@ -5533,7 +5524,6 @@ struct BatchOps {
         best = xch(*xplan);
         for (int w = 4; w <= 8; w *= 2) {
           const FusedState::XPlan p = x_shape(s->cm, h->n1, w);
-          if (p.wn == 0) continue;
           const float t = xch(p);
           if (t < margin * best) {
             best = t;

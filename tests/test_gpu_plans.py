@@ -1,0 +1,40 @@
+'''Which kernels a radial step takes: exchanges up to 256 cells, separate contractions above, where the exchange measured
+slower.
+'''
+import pytest
+
+from searay_amd import configs, uppe_kernel
+
+pytestmark = pytest.mark.gpu
+
+
+def _vol(nw, nr, share=1.0):
+    vol = configs.batched_radial(n=1, steps=200)[0][0]
+    vol['wave grid'] = (nw, nr, 1, 2)
+    vol['radial modes'] = nr
+    vol['nonlinear band'] = (0.0, share * vol['frequency band'][1])
+    return vol
+
+
+def _launches(vol, precision):
+    rs = uppe_kernel.RunSetup(vol)
+    zi, _, length = rs.plane(0)
+    with rs.make_stepper(uppe_kernel.hip_stepper_factory(precision)) as st:
+        st.set_field(rs.stepper_field())
+        st.profile_enable(True)
+        st.advance(zi, length, 0, rs.subcycles, rs.dzmin, max_steps=2)
+        return {c: st.profile_read(c)[1] for c in ('hankel', 'hankel_r2k', 'exchange')}
+
+
+@pytest.mark.parametrize('nw,precision', [(129, 'bf16x3'), (513, 'bf16x3'), (513, 'fp32'), (1025, 'fp64'),
+                                          (2049, 'fp64')])
+def test_tall_grids_take_separate_contractions(nw, precision):
+    print('plan of %d x 512 %s' % (nw, precision), flush=True)
+    assert _launches(_vol(nw, 512), precision) == {'hankel': 8, 'hankel_r2k': 8, 'exchange': 0}
+
+
+@pytest.mark.parametrize('nr', [8, 128, 256])
+@pytest.mark.parametrize('precision', ['fp64', 'fp32', 'bf16x3'])
+def test_other_grids_take_exchanges(nr, precision):
+    print('plan of 257 x %d %s' % (nr, precision), flush=True)
+    assert _launches(_vol(257, nr), precision) == {'hankel': 0, 'hankel_r2k': 0, 'exchange': 9}
