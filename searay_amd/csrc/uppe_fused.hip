@@ -1042,7 +1042,8 @@ __device__ inline void hankel_tile(
     // spills, half as much again (us per k2r launch: 2049 x 512 196 -> 122, 1025 x 1024 369 -> 226) and FP32 a twentieth
     // (2049 x 512 50.3 -> 47.8). FP32 has the registers for a second loop with a chunk's four rows at once. It pays while
     // the operator is small (us per k2r launch, one by one / at once: 4097 x 512 100 / 86; 2049 x 1024, whose operator is
-    // an XCD's L2, 190 / 200; 513 x 2048 198 / 203).
+    // an XCD's L2, 190 / 200; 513 x 2048 198 / 203). BF16x3, whose operands are half as many, has nothing to wait for and
+    // keeps one loop (with two 2049 x 256 took 129.1 us per step instead of 126.6).
     auto main_loop = [&](auto one) {
       constexpr bool ONE = decltype(one)::value;
       constexpr int NC = ONE ? 1 : CT;               // MFMA column tiles
@@ -1121,7 +1122,7 @@ __device__ inline void hankel_tile(
         }
       }
     };
-    constexpr bool two_loops = RT == 1 || CM == CM_F32;
+    constexpr bool two_loops = CM == CM_F32 || (CM == CM_F64 && RT == 1);
     if (two_loops && nmt == 1 && (RT == 1 || Kp <= 512)) {
       if constexpr (two_loops) main_loop(std::true_type());
     } else {
