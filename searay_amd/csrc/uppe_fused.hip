@@ -3930,11 +3930,18 @@ static FusedState::XPlan x_shape(int cm, int nr, int wn) {
 // O2 1025 x 128 201 / 173 / 169. Above 256 cells one tile's contractions hold a CU for longer than the separate
 // kernels, which split their rows over CUs (separate / 4 columns: BF16x3 129 x 512 116 / 124, 1025 x 512 165 / 203;
 // FP32 513 x 512 194 / 230; FP64 513 x 512 323 / 392, 1025 x 512 391 / 546, 2049 x 512 1016 / 1180).
+// Above 128 cells a tile holds a CU. A grid whose last nl tile, of a column or so, is one more than the CUs (all 2049
+// columns nonlinear) then takes two rounds where the separate kernels merge that column into their last tile and take
+// one (2049 x 256, fixed / adaptive steps, separate against 8 columns: BF16x3 128 / 132 against 141 / 158, FP32 186 /
+// 192 against 184 / 199, FP64 330 / 335 against 329 / 343; with 2048 nonlinear columns the exchange is ahead, BF16x3
+// 122 / 127 against 115 / 126). A launch of several instances merges nothing (4 x 513 x 256: 179 against 156).
 static FusedState::XPlan plan_exchange(int cm, int nr, int f1, int nw, int instances, int n_cu) {
   // SEARAY_UPPE_TILE_WIDTH pins the tiling of the separate contractions, so it asks for them
   if (cm < 0 || nr > 256 || getenv("SEARAY_UPPE_TILE_WIDTH")) return FusedState::XPlan();
   const int nlt = (f1 + 3) / 4, lin = (std::max(0, nw - 4 * nlt) + 7) / 8;
-  return x_shape(cm, nr, (long)(nlt + lin) * instances <= n_cu ? 4 : 8);
+  if ((long)(nlt + lin) * instances <= n_cu) return x_shape(cm, nr, 4);
+  if (instances == 1 && nr > 128 && (f1 + 7) / 8 > n_cu && nw / 8 <= n_cu) return FusedState::XPlan();
+  return x_shape(cm, nr, 8);
 }
 
 template <typename T>

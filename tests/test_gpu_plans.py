@@ -1,5 +1,5 @@
-'''Which kernels a radial step takes: exchanges up to 256 cells, separate contractions above, where the exchange measured
-slower.
+'''Which kernels a radial step takes: exchanges up to 256 cells, separate contractions above and where one tile more than
+the CUs would take a second round; there the exchange measured slower.
 '''
 import pytest
 
@@ -38,3 +38,14 @@ def test_tall_grids_take_separate_contractions(nw, precision):
 def test_other_grids_take_exchanges(nr, precision):
     print('plan of 257 x %d %s' % (nr, precision), flush=True)
     assert _launches(_vol(257, nr), precision) == {'hankel': 0, 'hankel_r2k': 0, 'exchange': 9}
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'fp32', 'bf16x3'])
+@pytest.mark.parametrize('columns,exchange', [(2049, False), (2048, True)])
+def test_one_tile_more_than_the_cus(precision, columns, exchange):
+    print('plan of 2049 x 256 %s, %d nonlinear columns' % (precision, columns), flush=True)
+    vol = _vol(2049, 256, (columns + 0.3) / 2049)
+    rs = uppe_kernel.RunSetup(vol)
+    assert rs.nl_filter[columns - 1] == 1.0 and not rs.nl_filter[columns:].any()
+    n = _launches(vol, precision)
+    assert (n['exchange'] > 0) == exchange and (n['hankel'] > 0) != exchange
