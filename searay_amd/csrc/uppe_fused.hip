@@ -5751,7 +5751,11 @@ void fused_batch_advance(uppe_batch* b, const uppe_step_control* c, int* steps_o
       r.count = j - r.first;
       r.plan[0] = h0->fused->plan[0];
       r.plan[1] = h0->fused->plan[1];
-      r.xplan = h0->fused->xplan;
+      // The exchange's tile width for the run's instances: narrow tiles of one grid are too many for several (16
+      // instances of 513 x 256, BF16x3, us per step: 450 with 4 columns, 364 with 8). The widths give equal results; the
+      // two kinds of contraction do so but in BF16x3, where a member takes the kind of a standalone handle.
+      if (h0->fused->xplan.wn > 0 || G.cm != CM_BF16X3)
+        r.xplan = plan_exchange(G.cm, h0->n1, h0->fused->f1, h0->nw, r.count, h0->fused->n_cu);
       r.known = true;
       for (int m = r.first; m < r.first + r.count; m++) r.known = r.known && G.st_host[m].fixed;
       r.spt = default_spt(h0, h0->fused, (long)r.count * h0->P);

@@ -47,3 +47,39 @@ def test_autotuned_batch_equals_standalone(nw, nr, nk, share, members, precision
             want = st.get_state()
         assert n == steps[i]
         assert np.array_equal(got[i], want), (i, tiles, np.max(np.abs(got[i] - want)) / np.max(np.abs(want)))
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'fp32', 'bf16x3'])
+def test_untuned_batches_plan_for_all_instances(precision):
+    nw, nr, nk, share, members = GRIDS[0]
+    vols = [_vol(nw, nr, nk, share, 0.5, False) for _ in range(members)]
+    f1 = int(np.nonzero(uppe_kernel.RunSetup(vols[0]).nl_filter)[0][-1]) + 1
+    tiles = []
+    for n in (2, members):
+        print('tiles of %d x %d x %d %s' % (n, nw, nr, precision), flush=True)
+        with batch.Batch(vols[:n], precision=precision, autotune=False) as b:
+            b.set_fields()
+            b.advance(max_steps=1)
+            tiles.append(b.plan(0)['r2k']['tiles'])
+    assert tiles == [(f1 + 3) // 4, (f1 + 7) // 8]
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'fp32'])
+@pytest.mark.parametrize('adaptive', [False, True])
+@pytest.mark.parametrize('nw,nr,nk,share,members', GRIDS)
+def test_exchange_equals_separate_contractions(nw, nr, nk, share, members, precision, adaptive, monkeypatch):
+    rs = uppe_kernel.RunSetup(_vol(nw, nr, nk, share, 1.0, adaptive))
+    zi, _, length = rs.plane(0)
+    states = []
+    for width in (None, '8'):  # a pinned width asks for the separate contractions
+        if width:
+            monkeypatch.setenv('SEARAY_UPPE_TILE_WIDTH', width)
+        print('exchange or not: %d x %d %s width %s' % (nw, nr, precision, width), flush=True)
+        with rs.make_stepper(uppe_kernel.hip_stepper_factory(precision)) as st:
+            st.set_field(rs.stepper_field())
+            st.profile_enable(True)
+            st.advance(zi, length, 0, rs.subcycles, rs.dzmin)
+            assert (st.profile_read('exchange')[1] > 0) == (width is None)
+            states.append(st.get_state())
+    scale = np.max(np.abs(states[0]))
+    assert np.max(np.abs(states[1] - states[0])) <= (1e-13 if precision == 'fp64' else 0.0) * scale
