@@ -5483,13 +5483,14 @@ struct BatchOps {
     return ms / reps;
   }
 
-  // choose launch shapes by timing on nz instances zs elements apart starting at member (h, s), as the second
-  // RK stage runs them: the k2r contraction with its stage prologue (writes E_r, scratch) and the r2k
-  // contraction with its stage epilogue (writes the second slope, which every step writes before it reads it)
-  // give the two plans; with src, the source kernel's samples per thread are timed too (it writes J_r,
-  // scratch). The state is not touched, and the plans do not change any result (every output sums its
-  // contraction in the same order). The incoming plans are the defaults: another candidate replaces one only
-  // when it is 3 % faster, so that timing noise does not pick between equals.
+  // choose launch shapes by timing on nz instances zs elements apart starting at member (h, s). Where the steps take
+  // the exchange, its tile width, as the second and third RK stages run it; otherwise the plans of the two separate
+  // contractions, as the second RK stage runs them. They write E_r, which is scratch, and the second and third slopes,
+  // which every step writes before it reads them. With src, the source kernel's samples per thread are timed too (it
+  // writes J_r, scratch). The state is not touched. The contraction plans do not change any result (every output sums
+  // its contraction in the same order); the samples per thread reorder the sums along a strip, so they are what an
+  // autotuned run's last bits depend on. The incoming plans are the defaults: another candidate replaces one only when
+  // it is 3 % faster, so that timing noise does not pick between equals.
   template <int CM>
   static void tune_shapes(uppe_handle* h, FusedState* s, int nz, long zs, const SrcInst* src,
                           FusedState::HkPlan plan[2], FusedState::XPlan* xplan, int* spt_out,
@@ -5522,7 +5523,7 @@ struct BatchOps {
       };
       // exchanges at a stage whose linear tiles run (3) and one whose do not (2)
       float best = 0.f;
-      if (xplan && xplan->wn > 0) {
+      if (xplan->wn > 0) {
         auto xch = [&](const FusedState::XPlan& p) {
           return time_launch(h->stream, e0, e1, [&] {
             F::template x_launch<CM>(h, s, p, (const C*)s->jr, (C*)s->er, 2, false, 1, nz, zs, share);
@@ -5540,7 +5541,7 @@ struct BatchOps {
         }
       }
       // the separate contractions, where the steps take them
-      if (!(xplan && xplan->wn > 0)) {
+      if (xplan->wn == 0) {
         // with the tile width pinned, the default plan is not a candidate: the first candidate is taken
         const bool pinned = getenv("SEARAY_UPPE_TILE_WIDTH") != nullptr;
         best = pinned ? 1e30f : k2r(plan[0]);
@@ -5627,10 +5628,10 @@ static int default_spt(const uppe_handle* h, const FusedState* s, long strips) {
 }
 
 // a standalone radial handle on the matrix cores: the source shape by default_spt; with SEARAY_UPPE_TUNE=1 the
-// contraction plans are also timed on the handle once per nonlinear band (the r2k plan depends on it). By
-// default a standalone handle keeps plan_hankel's plans, which fit one workgroup per CU: timing them against
-// the candidates on the single-instance workloads found no plan faster by more than the run-to-run spread, and
-// fixed plans keep every run's launch shapes (and the measured traffic per launch) the same.
+// plans its steps launch, of the exchange or of the separate contractions, are also timed on the handle once per
+// nonlinear band (they depend on it). By default a standalone handle keeps the plans of plan_exchange and
+// plan_hankel: timing them against the candidates on the single-instance workloads found no plan faster by more than
+// the run-to-run spread, and fixed plans keep every run's launch shapes (and the measured traffic per launch) the same.
 template <typename T>
 void tune_single(uppe_handle* h, FusedState* s, bool may_time) {
   if (s->cm < 0 || h->d.geometry != UPPE_RADIAL || s->tuned_f1 == s->f1) return;
@@ -5642,7 +5643,7 @@ void tune_single(uppe_handle* h, FusedState* s, bool may_time) {
   const char* env = getenv("SEARAY_UPPE_TUNE");
   if (env && env[0] == '1') {
     int unused = 0;
-    BatchOps<T>::tune_shapes(h, s, 1, 0, nullptr, s->plan, nullptr, &unused);
+    BatchOps<T>::tune_shapes(h, s, 1, 0, nullptr, s->plan, &s->xplan, &unused);
   }
   s->spt = default_spt(h, s, h->P);
   s->tuned_f1 = s->f1;

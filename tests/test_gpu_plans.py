@@ -1,6 +1,7 @@
 '''Which kernels a radial step takes: exchanges up to 256 cells, separate contractions above and where one tile more than
 the CUs would take a second round; there the exchange measured slower.
 '''
+import numpy as np
 import pytest
 
 from searay_amd import configs, uppe_kernel
@@ -49,3 +50,27 @@ def test_one_tile_more_than_the_cus(precision, columns, exchange):
     assert rs.nl_filter[columns - 1] == 1.0 and not rs.nl_filter[columns:].any()
     n = _launches(vol, precision)
     assert (n['exchange'] > 0) == exchange and (n['hankel'] > 0) != exchange
+
+
+@pytest.mark.parametrize('nr', [64, 512])
+@pytest.mark.parametrize('precision', ['fp64', 'fp32', 'bf16x3'])
+def test_tuned_handles_time_what_they_launch(nr, precision, monkeypatch):
+    '''SEARAY_UPPE_TUNE=1 times candidates of the launches that the steps take, and of no others, and changes no
+    result.'''
+    print('tuned handle 257 x %d %s' % (nr, precision), flush=True)
+    vol = _vol(257, nr)
+    rs = uppe_kernel.RunSetup(vol)
+    zi, _, length = rs.plane(0)
+    states, counts = [], []
+    for tune in ('0', '1'):
+        monkeypatch.setenv('SEARAY_UPPE_TUNE', tune)
+        with rs.make_stepper(uppe_kernel.hip_stepper_factory(precision)) as st:
+            st.set_field(rs.stepper_field())
+            st.profile_enable(True)
+            st.advance(zi, length, 0, rs.subcycles, rs.dzmin, max_steps=2)
+            counts.append({c: st.profile_read(c)[1] for c in ('hankel', 'hankel_r2k', 'exchange')})
+            states.append(st.get_state())
+    taken = {c for c, n in counts[0].items() if n > 0}
+    assert {c for c, n in counts[1].items() if n > counts[0][c]} == taken
+    assert all(counts[1][c] == 0 for c in counts[1] if c not in taken)
+    assert np.array_equal(states[0], states[1])
