@@ -5146,15 +5146,6 @@ struct Fused {
       gemm_once<PRO_FINISH>(h, s, (const T*)s->Hb, (const C*)s->q, (C*)s->er, h->n1, h->nk, z_total, s->qbase, s->f1);
       azim(h, s, (C*)s->er, h->nw, +1);
     }
-    const bool diag = j_r || chi_t || ne_t;  // the field alone needs no source
-    if (diag && h->paraxial) {
-      // the envelope source takes A itself (paraxial_kernel.py:243-245)
-      source(h, s, (const C*)s->er, (C*)s->jr, true, nullptr);
-    } else if (diag) {
-      UPPE_HIP(hipMemcpyAsync(s->k1, s->er, sizeof(C) * n, hipMemcpyDeviceToDevice, h->stream));
-      launchf(h, UPPE_KC_POINT, f_vp_to_e<T>, dim3(grid_for(n)), dim3(kBlock), 0, (C*)s->k1, (const C*)s->kzc, n);
-      source(h, s, (const C*)s->k1, (C*)s->jr, true, nullptr);
-    }
     auto out_c = [&](const void* src, double* dst) {
       launchf(h, UPPE_KC_POINT, f_to_host<T>, dim3(grid_for(P * h->nw)), dim3(kBlock), 0, (const C*)src, s->stage,
               h->nw, P, s->nwp, (const C*)nullptr, 0, 0.0);
@@ -5168,11 +5159,16 @@ struct Fused {
       UPPE_HIP(hipStreamSynchronize(h->stream));
     };
     if (a_r) out_c(s->er, a_r);
+    if (j_r || chi_t || ne_t) {  // the field alone needs no source
+      // E = i kz A in place; the envelope source takes A itself (paraxial_kernel.py:243-245). The stage buffers stay as
+      // they are: forming E in one of them took a copy and a clear, 10 us of a small grid's 120.
+      if (!h->paraxial)
+        launchf(h, UPPE_KC_POINT, f_vp_to_e<T>, dim3(grid_for(n)), dim3(kBlock), 0, (C*)s->er, (const C*)s->kzc, n);
+      source(h, s, (const C*)s->er, (C*)s->jr, true, nullptr);
+    }
     if (j_r) out_c(s->jr, j_r);
     if (chi_t) out_t(s->chi_t, chi_t);
     if (ne_t) out_t(s->ne_t, ne_t);
-    // the diagnostics leave k1 holding the r-space field: clear it so the next run starts from zero stage buffers
-    if (diag) UPPE_HIP(hipMemsetAsync(s->k1, 0, sizeof(C) * n, h->stream));
     UPPE_HIP(hipStreamSynchronize(h->stream));
   }
 
