@@ -4702,10 +4702,18 @@ struct Fused {
             h->paraxial ? 1 : 0);
   }
 
+  // Whether a grid takes its y passes in exchanges. An FP64 grid with long lines and few workgroups does not: its double
+  // sines and exponentials run faster in the two launches (us per step, two launches / one: 17 x 2 x 256, 6 workgroups,
+  // 161 / 169; 33 x 8 x 1024, 40, 348 / 431; 65 x 8 x 1024, 72, 359 / 343; 65 x 8 x 256, 72, 175 / 153; 17 x 2 x 64
+  // 123 / 117; FP32 17 x 2 x 1024 150 / 125).
+  static bool takes_texch(const uppe_handle* h, const FusedState* s) {
+    return sizeof(T) == 4 || h->n2 < 256 || 4L * ((h->nw + 7) / 8) * h->n1 >= s->n_cu;
+  }
+
   // One RK4 step on a Cartesian grid: per RHS, the x pass of the inverse transform, the source, the x pass of the
   // forward transform over the nonlinear band, and the y passes of the forward and of the next stage's inverse
   // transform in one launch. `first` and `known` as for step_mfma: a run opens with a y pass of its own, and an
-  // adaptive one takes stage 1's y passes one by one.
+  // adaptive one takes stage 1's y passes one by one, as a grid that takes no exchanges does at every stage.
   static void step_cart(uppe_handle* h, FusedState* s, bool first, bool known) {
     const C* kp[5] = {nullptr, nullptr, (const C*)s->k1, (const C*)s->k2, (const C*)s->k3};
     C *q = (C*)s->q, *er = (C*)s->er, *jr = (C*)s->jr;
@@ -4715,14 +4723,15 @@ struct Fused {
       else
         tpass<PRO_STAGE, EPI_NONE>(h, s, 2, q, er, h->nw, +1, kp[stage], stage, 0.0, s->st);
     };
-    if (first) open(1);
+    const bool x = takes_texch(h, s);
+    if (first || !x) open(1);
     for (int stage = 1; stage <= 4; stage++) {
       tpass<PRO_NONE, EPI_NONE>(h, s, 1, er, er, h->nw, +1, nullptr, stage, 0.0, s->st);
       source(h, s, er, jr, false, stage == 1 ? s->st : nullptr);
       tpass<PRO_NONE, EPI_NONE>(h, s, 1, jr, jr, s->f1, -1, nullptr, stage, 0.0, s->st);
-      if (stage == 1 && !known) {
+      if (!x || (stage == 1 && !known)) {
         tpass<PRO_NONE, EPI_STAGE>(h, s, 2, jr, (C*)nullptr, s->f1, -1, nullptr, stage, 0.0, s->st);
-        open(2);
+        if (stage < 4) open(stage + 1);
         continue;
       }
       if constexpr (sizeof(T) == 4) {
