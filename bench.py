@@ -13,7 +13,7 @@ Printed JSON line (one):
                 dispatch-stamped HIP events on every launch) against HBM bandwidth: its algorithmic bytes per
                 launch over its average launch duration. Per grid point in FP32: k->r contraction 28 B, source 16 B,
                 r->k contraction 52 B over the nonlinear band's columns (96 B per right-hand side); doubled in FP64.
-                A contraction is also reported against the matrix-core peak of the type it issues. `traffic` (HBM
+                An exchange of the two counts what the launches of a step read and write on their average. A contraction is also reported against the matrix-core peak of the type it issues. `traffic` (HBM
                 bytes per launch, rocprofv3 FETCH_SIZE and WRITE_SIZE, copy-calibrated) and `mfma_busy_frac` come
                 from the committed counter summary of the same kernel and workload (profiles/counters_*.json) when
                 there is one. `per_kernel` lists every step kernel's average duration and share
@@ -78,12 +78,32 @@ def nl_columns(rs):
     return int(min(rs.N[0], max((nz[-1] + 1) if nz.size else 0, 4)))
 
 
-def kernel_work(rs, kernel, el, prec):
+def exchange_work(nw, f1, nr, nk, el, prec, adaptive):
+    '''Algorithmic bytes and MFMA flops of one exchange launch, averaged over the launches of a step inside a subcycle
+    (4, or 5 when adaptive). A complex value is 2 el bytes, the phase table 8 bytes a point.
+
+    The f1 columns of the nonlinear band: J_r in and E_r out at every stage; per point the phase, kz and q at every
+    stage, the slope out at stages 1 to 3, three slopes in and q out at stage 4. An adaptive step opens stage 2 in a
+    launch of its own, which reads the phase, kz, q and the first slope again. The columns above it: the phase, kz and q
+    in and E_r out where their phase coordinate moves, from stage 1 to 2 and from 3 to 4. Both contractions run over the
+    band at every stage, the second one alone over the other columns at those two stages: 4 N_cols Nk Nr flops each, in
+    BF16x3 times the four partial products.'''
+    c, launches = 2.0 * el, 5 if adaptive else 4
+    state = 8.0 + 2 * c
+    band, rest = f1, nw - f1
+    per_step = band * nr * 8 * c + band * nk * (4 * state + 3 * c + 4 * c) + rest * 2 * (nk * state + nr * c)
+    if adaptive:
+        per_step += band * nk * (state + c)
+    flops = 4.0 * nk * nr * (4 * 2 * band + 2 * rest) * (4.0 if prec == 'bf16x3' else 1.0)
+    return per_step / launches, flops / launches
+
+
+def kernel_work(rs, kernel, el, prec, adaptive=False):
     '''Algorithmic bytes and MFMA flops (as issued) of one launch of a radial step kernel. Per grid point in FP32:
     k->r 28 B (the stage input in, E_r out: 16 B, plus 12 B of kz tables), source 16 B (E_r in, J_r out), r->k 52 B
     (J_r in and the RK stage: 40 B, plus the tables) over the columns of the nonlinear band only; 96 B per RHS in
-    all. An exchange does both contractions with one read of the state and tables: the r->k bytes and E_r out. FP64
-    doubles them. The contractions issue 4 N_cols Nk Nr flops, three times that in BF16x3.'''
+    all. FP64 doubles them. The contractions issue 4 N_cols Nk Nr flops, three times that in BF16x3. An exchange does
+    both contractions with one read of the state and tables (exchange_work).'''
     T = rs.field_tool.GetTransverseTool()
     nw, nr, nk = rs.N[0], rs.N[1], getattr(T, 'Nk', rs.N[1])
     scale = el / 4.0
@@ -94,8 +114,7 @@ def kernel_work(rs, kernel, el, prec):
         f1 = nl_columns(rs)
         return 52.0 * scale * f1 * nk, 4.0 * f1 * nk * nr * issued
     if kernel == 'exchange':
-        f1 = nl_columns(rs)
-        return scale * (52.0 * f1 * nk + 8.0 * nw * nr), 4.0 * (f1 + nw) * nk * nr * issued
+        return exchange_work(nw, nl_columns(rs), nr, nk, el, prec, adaptive)
     if kernel == 'source':
         return 16.0 * scale * nw * nr, 0.0
     return None, None
@@ -130,7 +149,9 @@ def roofline_of(rs, prec, classes, ms_per_step, counters=None):
     dom = max(timed, key=lambda k: timed[k][0])
     ms, cnt = timed[dom]
     avg_s = ms / cnt * 1e-3
-    B, F = kernel_work(rs, dom, el, prec)
+    # one exchange opens the run; then an adaptive step takes five to its four sources
+    adaptive = classes.get('exchange', (0, 0))[1] - 1 > 1.125 * classes.get('source', (0, 0))[1]
+    B, F = kernel_work(rs, dom, el, prec, adaptive)
     achieved = B / avg_s / 1e9
     traffic = None
     extra = {}
@@ -150,7 +171,7 @@ def roofline_of(rs, prec, classes, ms_per_step, counters=None):
     for k, (kms, kn) in classes.items():
         if kn == 0:
             continue
-        b, _ = kernel_work(rs, k, el, prec)
+        b, _ = kernel_work(rs, k, el, prec, adaptive)
         a = kms / kn * 1e-3
         per_kernel[k] = dict(avg_launch_us=a * 1e6, launches=kn, share=round(kms / total, 4),
                              achieved_gbs=(b / a / 1e9) if b else None)
