@@ -12,7 +12,9 @@
 //      P, J_p -> one complex FFT for both rffts -> spectral current and filter (uppe_kernel.py:139-186);
 //   3. r2k GEMM; its epilogue forms the ODE right-hand side (uppe.cl:73-91) and the RK bookkeeping, the
 //      per-point step estimate (paraxial.cl:40-58) and the field conditioner (uppe_kernel.py:131-137).
-// Step control (uppe_kernel.py:218-227, 299-325) runs on the device inside these three launches (step_pos,
+// Between right-hand sides, radial grids up to 256 cells take 3 of a stage and 1 of the next in one launch (f_exchange),
+// and Cartesian grids the last pass of 3 and the first of 1 (f_texch).
+// Step control (uppe_kernel.py:218-227, 299-325) runs on the device inside these launches (step_pos,
 // step_commit), so a whole subcycle runs without host synchronisation and without launches of its own.
 #include <hip/hip_ext.h>
 
@@ -230,8 +232,9 @@ __device__ inline int red_slot(int block) { return (block & (kSlots - 1)) * kSlo
 // step state. The step size is a function of the committed state (stage 1's r2k epilogue leaves the minimum
 // per-point estimate in dzraw), so every launch from stage 2 on forms it itself. The end of a step (z advance,
 // subcycle bookkeeping, records) is committed by the first block of the next step's stage-1 source launch, which
-// is the first launch that reads nothing of the state; until then the step is marked pending, and the next
-// step's stage-1 k2r launch advances a local copy. A chunk of steps ends with one commit launch (f_ctl_commit).
+// is the first launch that reads nothing of the state; until then the step is marked pending. Whichever launch forms the
+// next step's stage-1 field before that advances a local copy: the exchange of stage 4, or the next step's stage-1 k2r
+// launch. A chunk of steps ends with one commit launch (f_ctl_commit).
 // ---------------------------------------------------------------------------------------------------
 
 // dz of the current step: the replayed schedule, the subcycle's remainder for fixed steps, or the estimate
@@ -3592,7 +3595,6 @@ __global__ void f_fill_zero(unsigned long long* p, long n) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) p[i] = 0ull;
 }
 
-// max |q| over the state (set_field)
 // max|q| over P rows of columns [f_all, nwp) into all and over columns [f_from, nwp) into part (f_all <= f_from): a
 // block takes whole rows and adds one value to each word (a word takes an atomic every 12 ns: one per wavefront of 256
 // blocks cost 13 us, whatever the field)
@@ -3625,6 +3627,7 @@ __global__ __launch_bounds__(256) void f_qmax(const cplx<T>* q, long P, int nwp,
   }
 }
 
+// host layout (nw, P) complex128 -> [P][nwp] complex T (zero padding)
 template <typename T>
 __global__ void f_from_host(const double* src, cplx<T>* dst, int nw, long P, int nwp) {
   long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
@@ -4309,10 +4312,9 @@ struct Fused {
     UPPE_HIP(hipStreamSynchronize(h->stream));
   }
 
-  // SIMT contraction (the one-off transforms of set_field/finish): one launch per azimuthal mode m over the rows
-  // r N2 + m, with that mode's operator
-  // a transform outside the steps: every azimuthal mode's out = A in. 16-row tiles while 64-row ones are fewer than
-  // four per CU (FP32) or one (FP64, where every row tile repeats the prologue's double sines and exponentials)
+  // a transform outside the steps (set_field, finish): out = A in on the vector units, one launch per azimuthal mode m
+  // over the rows r N2 + m, with that mode's operator. 16-row tiles while 64-row ones are fewer than four per CU (FP32)
+  // or one (FP64, where every row tile repeats the prologue's double sines and exponentials)
   template <int PRO>
   static void gemm_once(uppe_handle* h, FusedState* s, const T* A, const C* in, C* out, int M, int K, double z,
                         double qbase, int f1) {
@@ -4656,7 +4658,6 @@ struct Fused {
     }
   }
 
-  // one RK4 step: 4 x (k2r, source, r2k); the step control runs inside them
   // one 1-D pass of a Cartesian transverse transform over columns [0, fend); sign +1 inverse (scaled 1/Na).
   // CW columns per line: 128-byte runs (16 FP32 or 8 FP64 columns), 8 FP32 columns for lines of 1024 points
   // (the block holds CW Na/8 <= 1024 threads)
