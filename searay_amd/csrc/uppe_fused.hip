@@ -3947,6 +3947,18 @@ static FusedState::XPlan plan_exchange(int cm, int nr, int f1, int nw, int insta
   return x_shape(cm, nr, 8);
 }
 
+// Whether a batch run of many instances is better served by separate contractions, once their plans are timed: their
+// wide tiles and row blocks read an operator less often than exchange tiles do, which counts when the tiles take several
+// rounds of the device's waves. us per step, separate with timed plans / exchange: BF16x3 at 2.03 rounds 16 x 513 x 128
+// 175 / 186, 8 x 513 x 256 215 / 230, at 8 16 x 1025 x 256 513 / 610, at 1.5 12 x 513 x 128 152 / 151, with small
+// operators 64 x 257 x 64 174 / 164; FP32 at 4.1 rounds 16 x 513 x 256 455 / 464, 32 x 257 x 256 441 / 460, at 8 16 x
+// 1025 x 256 756 / 773, at 4 8 x 1025 x 256 436 / 422. FP64 stays with the exchange (16 x 1025 x 256 1677 / 1470).
+static bool batch_prefers_separate(int cm, int nr, int f1, int instances, int n_cu) {
+  if (cm == CM_F64 || nr <= (cm == CM_BF16X3 ? 64 : 128)) return false;
+  const long waves = (long)((f1 + 7) / 8) * instances * ((nr + 15) / 16);
+  return waves > (cm == CM_BF16X3 ? 2L : 4L) * 16 * n_cu;
+}
+
 template <typename T>
 void tune_single(uppe_handle* h, FusedState* s, bool may_time = true);
 
@@ -5760,8 +5772,10 @@ void fused_batch_advance(uppe_batch* b, const uppe_step_control* c, int* steps_o
       r.plan[1] = h0->fused->plan[1];
       // The exchange's tile width for the run's instances: narrow tiles of one grid are too many for several (16
       // instances of 513 x 256, BF16x3, us per step: 450 with 4 columns, 364 with 8). The widths give equal results; the
-      // two kinds of contraction do so but in BF16x3, where a member takes the kind of a standalone handle.
-      if (h0->fused->xplan.wn > 0 || G.cm != CM_BF16X3)
+      // two kinds of contraction do so but in BF16x3, where members take the kind of a standalone handle unless the
+      // plans are timed.
+      if ((h0->fused->xplan.wn > 0 || G.cm != CM_BF16X3) &&
+          !(fb->autotune && batch_prefers_separate(G.cm, h0->n1, h0->fused->f1, r.count, h0->fused->n_cu)))
         r.xplan = plan_exchange(G.cm, h0->n1, h0->fused->f1, h0->nw, r.count, h0->fused->n_cu);
       r.known = true;
       for (int m = r.first; m < r.first + r.count; m++) r.known = r.known && G.st_host[m].fixed;

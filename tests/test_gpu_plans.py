@@ -4,7 +4,7 @@ the CUs would take a second round; there the exchange measured slower.
 import numpy as np
 import pytest
 
-from searay_amd import configs, uppe_kernel
+from searay_amd import batch, configs, uppe_kernel
 
 pytestmark = pytest.mark.gpu
 
@@ -74,3 +74,32 @@ def test_tuned_handles_time_what_they_launch(nr, precision, monkeypatch):
     assert {c for c, n in counts[1].items() if n > counts[0][c]} == taken
     assert all(counts[1][c] == 0 for c in counts[1] if c not in taken)
     assert np.array_equal(states[0], states[1])
+
+
+@pytest.mark.parametrize('nr,members,precision,autotune,exchange', [
+    (128, 16, 'bf16x3', True, False), (128, 16, 'bf16x3', False, True), (128, 12, 'bf16x3', True, True),
+    (64, 32, 'bf16x3', True, True), (256, 16, 'fp32', True, False), (256, 8, 'fp32', True, True),
+    (256, 16, 'fp64', True, True)])
+def test_large_tuned_batches_take_separate_contractions(nr, members, precision, autotune, exchange):
+    print('plan of %d x 513 x %d %s autotune=%s' % (members, nr, precision, autotune), flush=True)
+    vols = configs.batched_radial(n=members, scale=2, steps=200)[0]
+    for vol in vols:
+        vol['wave grid'] = (513, nr, 1, 2)
+        vol['radial modes'] = nr
+    with batch.Batch(vols, precision=precision, autotune=autotune) as b:
+        b.set_fields()
+        b.advance(max_steps=1)  # times the plans
+        b.set_fields()
+        b.members[0].profile_enable(True)
+        b.advance(max_steps=2)
+        assert b.plan(0)['run_length'] == members
+        n = {c: b.members[0].profile_read(c)[1] for c in ('hankel', 'hankel_r2k', 'exchange')}
+        q = b.members[members - 1].get_state()
+    assert (n['exchange'] > 0) == exchange and (n['hankel_r2k'] > 0) != exchange
+    rs = uppe_kernel.RunSetup(vols[-1])
+    zi, _, length = rs.plane(0)
+    with rs.make_stepper(uppe_kernel.hip_stepper_factory(precision)) as st:
+        st.set_field(rs.stepper_field())
+        st.advance(zi, length, 0, rs.subcycles, rs.dzmin, max_steps=2)
+        want = st.get_state()
+    assert np.linalg.norm(q - want) < (1e-12 if precision == 'fp64' else 1e-5) * np.linalg.norm(want)
