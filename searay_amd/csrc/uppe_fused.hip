@@ -3954,7 +3954,7 @@ static FusedState::XPlan plan_exchange(int cm, int nr, int f1, int nw, int insta
 // operators 64 x 257 x 64 174 / 164; FP32 at 4.1 rounds 16 x 513 x 256 455 / 464, 32 x 257 x 256 441 / 460, at 8 16 x
 // 1025 x 256 756 / 773, at 4 8 x 1025 x 256 436 / 422. FP64 stays with the exchange (16 x 1025 x 256 1677 / 1470).
 static bool batch_prefers_separate(int cm, int nr, int f1, int instances, int n_cu) {
-  if (cm == CM_F64 || nr <= (cm == CM_BF16X3 ? 64 : 128)) return false;
+  if (cm == CM_F64 || instances < 2 || nr <= (cm == CM_BF16X3 ? 64 : 128)) return false;
   const long waves = (long)((f1 + 7) / 8) * instances * ((nr + 15) / 16);
   return waves > (cm == CM_BF16X3 ? 2L : 4L) * 16 * n_cu;
 }
